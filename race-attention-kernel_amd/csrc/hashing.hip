@@ -292,6 +292,8 @@ size_t hash_lds_bytes(int dk, int L, int K) {
 
 hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, int64_t rows,
                             int dk, int L, int K, int dtype, hipStream_t stream) {
+    if (hash_rows_supported(x, probs, probs, dk, L, K, dtype))
+        return launch_hash_rows(x, planes_T, nullptr, probs, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kHashRows - 1) / kHashRows));
     const size_t lds = hash_lds_bytes(dk, L, K);
     const bool vec = dk % 4 == 0;
@@ -324,6 +326,8 @@ hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, 
 
 hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const void* dprobs, void* dx,
                                 int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream) {
+    if (hash_rows_supported(x, dprobs, dx, dk, L, K, dtype))
+        return launch_hash_rows(x, planes_T, dprobs, dx, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kThreads - 1) / kThreads));
     const int tier = lk_tier(L * K);
     const size_t lds = size_t(dk) * tier * sizeof(float);

@@ -338,6 +338,13 @@ hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, 
 hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const void* dprobs, void* dx,
                                 int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream);
 
+// The same two on the matrix cores, 16 rows per wave (hash_rows.hip): whether
+// these arrays and this shape have kernels there, and the launch (dprobs null:
+// probs into `out`; else dx into `out`).
+bool hash_rows_supported(const void* x, const void* probs, const void* dx, int dk, int L, int K, int dtype);
+hipError_t launch_hash_rows(const void* x, const float* planes_T, const void* dprobs, void* out, int64_t rows,
+                            int dk, int L, int K, int dtype, hipStream_t stream);
+
 // ---- Algorithm 1 with the hashing inside (alg1.hip): bf16 q, k, v, out ----
 struct Alg1Args {
     const void* q;

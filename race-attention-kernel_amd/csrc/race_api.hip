@@ -189,10 +189,34 @@ FwdLayout fwd_layout(const Problem& p, int causal) {
     return l;
 }
 
+// Whether the non-causal passes run on the fp32 matrix cores: widths that are
+// multiples of 4, unless the vector ALU is asked for.
+bool nc_matrix_cores(const Problem& p) { return p.kernel != RACE_KERNEL_VALU && v4_widths(p.S, p.d); }
+
+// Token chunks of the non-causal reductions on the matrix cores, one record
+// each.  An explicit tile length is the chunk; the automatic one splits each
+// stream evenly into the blocks that suit the launch (nc_blocks_per_stream),
+// so that the maps have few records to add.  Never more chunks than tiles: the
+// workspace is sized for the tiles.
+Problem nc_chunks(const Problem& p, const race_options* o) {
+    if (!nc_matrix_cores(p) || (o && o->tile_tokens != 0) || p.N == 0 || p.T == 0) return p;
+    Problem c = p;
+    int64_t per = nc_blocks_per_stream(p.N, p.T, p.dtype, kMaxAutoTileOther);
+    if (per > p.tiles) per = p.tiles;
+    c.tile = int(((p.T + per - 1) / per + 15) / 16 * 16);
+    c.tiles = (p.T + c.tile - 1) / c.tile;
+    return c;
+}
+
 // Non-causal forwards with at most this many tiles per stream sum the tile
 // records as the map stages its matrix (every map workgroup of a stream sums
-// them again); longer ones reduce them once into E first.
+// them again); longer ones reduce them once into E first, and the backward
+// finalizes them.  The chunks the library chooses itself on the matrix cores
+// fold up to kNcFoldParts.
 constexpr int64_t kFoldTiles = 4;
+int64_t nc_fold(const Problem& p, const race_options* o) {
+    return nc_matrix_cores(p) && (!o || o->tile_tokens == 0) ? kNcFoldParts : kFoldTiles;
+}
 
 struct BwdLayout {
     int64_t records = 0, dB = 0, dA = 0;
@@ -361,16 +385,19 @@ hipError_t max_lds(int* bytes) {
 }
 
 
-// The non-causal reduction and map: the 16-byte-vector kernels when both
-// widths are multiples of 4, the scalar ones otherwise.
+// The non-causal reduction and map.  Widths that are multiples of 4 run on
+// the fp32 matrix cores, or with RACE_KERNEL_VALU on the 16-byte-vector ALU
+// kernels; other widths take the scalar kernels.
 hipError_t outer_sums(const void* x, const void* y, float* records, const Problem& p, int Wa,
                       int Wb, hipStream_t stream) {
+    if (nc_matrix_cores(p)) return launch_nc_sums(x, y, records, p, Wa, Wb, stream);
     if (v4_widths(Wa, Wb)) return launch_outer_sums4(x, y, records, p, Wa, Wb, stream);
     return launch_tile_outer_sums(x, y, records, p, Wa, Wb, stream);
 }
 
 hipError_t token_map(const void* x, void* out, const MapOperand& op, const Problem& p, int Wa,
                      int Wb, hipStream_t stream) {
+    if (nc_matrix_cores(p)) return launch_nc_map(x, out, op, p, Wa, Wb, stream);
     if (v4_widths(Wa, Wb)) return launch_map4(x, out, op, p, Wa, Wb, stream);
     return launch_token_map(x, out, op, p, Wa, Wb, stream);
 }
@@ -506,11 +533,12 @@ race_status fwd_impl(const void* probsQ, const void* probsK, const void* V, void
         return marks->mark(stream);
     }
 
+    p = nc_chunks(p, opts);
     RACE_TRY(marks->mark(stream));
     RACE_TRY(outer_sums(probsK, V, records, p, p.S, p.d, stream));
     RACE_TRY(marks->mark(stream));
     const int64_t Sd = int64_t(p.S) * p.d;
-    if (p.tiles > kFoldTiles) {
+    if (p.tiles > nc_fold(p, opts)) {
         float* E = records + l.records;
         RACE_TRY(launch_tile_reduce(records, state, E, p, stream));
         RACE_TRY(marks->mark(stream));
@@ -607,8 +635,35 @@ race_status noncausal_bwd_impl(const void* probsQ, const void* probsK, const voi
     float* dA = dB + l.dB;
     const int64_t Sd = int64_t(p.S) * p.d;
     const int64_t state_stride = Sd + p.S;
+    p = nc_chunks(p, opts);
 
     RACE_TRY(marks->mark(stream));
+    // S = d = 64 on the matrix cores: the query side (dQ and the dE records,
+    // dOut read once; a part that is not asked for runs as its own pass, with
+    // the same sums), then the key side.
+    if (p.S == 64 && p.d == 64 && nc_matrix_cores(p)) {
+        if (dQ && (dK || dV)) {
+            RACE_TRY(launch_nc_query64(probsQ, dOut, dQ, state, records, p, stream));
+        } else if (dQ) {
+            MapOperand op = map_operand(state, state_stride, 1, p.d);
+            op.div = state + Sd;
+            op.div_stream = state_stride;
+            op.div_by_col = true;
+            RACE_TRY(launch_nc_map(dOut, dQ, op, p, p.d, p.S, stream));
+        } else {
+            RACE_TRY(launch_nc_sums(probsQ, dOut, records, p, p.S, p.d, stream));
+        }
+        RACE_TRY(marks->mark(stream));
+        if (!dK && !dV) return RACE_SUCCESS;
+        if (p.tiles <= nc_fold(p, opts)) {
+            RACE_TRY(launch_nc_key64(probsK, V, dK, dV, records, state, nullptr, nullptr, p, stream));
+        } else {
+            RACE_TRY(launch_bwd_finalize(records, state, dB, dA, p, stream));
+            RACE_TRY(marks->mark(stream));
+            RACE_TRY(launch_nc_key64(probsK, V, dK, dV, nullptr, nullptr, dB, dA, p, stream));
+        }
+        return marks->mark(stream);
+    }
     // S = d = 64: the query side (dQ and the dE records, dOut read once) and,
     // with both dK and dV asked for, the key side each in one pass; the key
     // side forms dB and dA itself from up to kKeyGradFoldParts records per

@@ -167,6 +167,26 @@ hipError_t launch_key_grad64(const void* k, const void* v, void* dk, void* dv,
                              const float* dE_records, const float* state, const float* dB_ready,
                              const float* dA_ready, const Problem& p, hipStream_t stream);
 
+// ---- the same passes on the fp32 matrix cores (noncausal_mfma.hip), for the
+// same widths: fp32 products and sums, token operands straight from memory ----
+
+// Tile records a map or a key side sums as it stages its matrix; longer
+// sequences reduce them first.
+constexpr int kNcFoldParts = 8;
+// Workgroups per stream of those passes for `streams` streams of T tokens.
+int64_t nc_blocks_per_stream(int64_t streams, int64_t T, int dtype, int64_t max_tokens);
+hipError_t launch_nc_sums(const void* x, const void* y, float* records, const Problem& p, int Wa, int Wb,
+                          hipStream_t stream);
+hipError_t launch_nc_map(const void* x, void* out, const MapOperand& op, const Problem& p, int Wa, int Wb,
+                         hipStream_t stream);
+// S = d = 64: the query side and the key side (dk or dv may be null; dB_ready
+// and dA_ready past kNcFoldParts tiles per stream).
+hipError_t launch_nc_query64(const void* q, const void* g, void* dq, const float* state, float* records,
+                             const Problem& p, hipStream_t stream);
+hipError_t launch_nc_key64(const void* k, const void* v, void* dk, void* dv, const float* dE_records,
+                           const float* state, const float* dB_ready, const float* dA_ready, const Problem& p,
+                           hipStream_t stream);
+
 // ---- causal backward (causal_bwd.hip): fp32 vector-ALU kernels ----
 
 // Sub-chunk length (32 or 16) of the causal backward kernels for (S, d) under

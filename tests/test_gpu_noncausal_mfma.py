@@ -1,0 +1,102 @@
+"""The non-causal reductions and maps on the fp32 matrix cores.
+
+Widths that fill and that only part-fill the 16-lane vectors, the 16-column
+blocks, the 64-column slices and the bf16 operands of eight values (bf16 rows
+of 8 m + 4 values are widened to fp32), token counts around the 16- and
+32-token steps, and every way the tile records are added (by the maps, by the
+separate reduce and finalize), against fp64; the vector-ALU kernels
+(kernel="valu") of the same widths under the same bounds.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+EPS = 1e-6
+
+
+def exact(q, k, v, g):
+    """out, dQ, dK, dV in fp64, and for each the sum of its terms' magnitudes."""
+    N, T = q.shape[:2]
+    q, k = q.reshape(N, T, -1).double(), k.reshape(N, T, -1).double()
+    v, g = v.double(), g.double()
+    A = k.sum(1) + EPS
+
+    def grads(q, k, v, g, sign):
+        E = k.transpose(1, 2) @ v / A[..., None]
+        dE = q.transpose(1, 2) @ g
+        dB = dE / A[..., None]
+        dA = sign * (dE * E).sum(-1) / A
+        return (q @ E, g @ E.transpose(1, 2), v @ dB.transpose(1, 2) + dA[:, None], k @ dB)
+
+    return grads(q, k, v, g, -1.0), grads(q, k, v.abs(), g.abs(), 1.0)
+
+
+def check(got, want, scale, T, S, d, dtype, label):
+    # Every value is a sum of products of sums: at most T + S + d roundings of
+    # the terms' magnitudes in each of the three nested sums, and a few more
+    # from the divisions; bf16 outputs are rounded once.
+    rel = 3 * (T + S + d + 16) * U
+    for name, a, w, s in zip(("out", "dQ", "dK", "dV"), got, want, scale):
+        if a is None:
+            continue
+        err = (a.reshape(w.shape).double().cpu() - w).abs()
+        bound = rel * s + (2.0 ** -8 * w.abs() if dtype == torch.bfloat16 else 0.0) + 1e-30
+        assert bool((err <= bound).all()), (label, name, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L, R, d", [(1, 4, 4), (3, 4, 20), (2, 8, 64), (3, 16, 96), (5, 20, 36), (4, 16, 64),
+                                     (8, 16, 128), (17, 12, 100), (8, 32, 128)])
+@pytest.mark.parametrize("N, T", [(2, 1), (3, 33), (2, 130), (2, 1100), (130, 70)])
+def test_widths_and_lengths(race, cuda, dtype, L, R, d, N, T):
+    say("nc-mfma", dtype, L, R, d, N, T)
+    q, k, v, g = race.make_inputs(N, T, L, R, d, seed=N + T + d, dtype=dtype, grad_out=True)
+    leaves = [x.to(cuda).requires_grad_(True) for x in (q, k, v)]
+    out = race.race_fused_fwd(*leaves, causal=False)
+    grads = torch.autograd.grad(out, leaves, g.to(cuda))
+    want, scale = exact(q, k, v, g)
+    check((out, *grads), want, scale, T, L * R, d, dtype, "mfma")
+    valu = race.race_fused_fwd(*(x.detach() for x in leaves), causal=False, kernel="valu")
+    check((valu, None, None, None), want, scale, T, L * R, d, dtype, "valu")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tile", [0, 64, 128, 1024])
+def test_records_added_by_the_maps_or_before_them(race, cuda, dtype, tile):
+    # T = 500: 8 tiles of 64 and 4 of 128 (separate reduce and finalize; the
+    # maps), 1 of 1024, and the automatic chunks.
+    N, T, L, R, d = 3, 500, 4, 16, 64
+    q, k, v, g = race.make_inputs(N, T, L, R, d, seed=5, dtype=dtype, grad_out=True)
+    qc, kc, vc, gc = (x.to(cuda) for x in (q, k, v, g))
+    out, state = race.race_fused_fwd_with_state(qc, kc, vc, causal=False, tile_tokens=tile)
+    want, scale = exact(q, k, v, g)
+    full = race.race_noncausal_backward(qc, kc, vc, gc, state, tile_tokens=tile)
+    check((out, *full), want, scale, T, L * R, d, dtype, tile)
+    B = torch.einsum("nts,ntc->nsc", k.reshape(N, T, -1).double(), v.double()).reshape(N, -1)
+    np.testing.assert_allclose(state[:, :-64].double().cpu().numpy(), B.numpy(), atol=T * U * 2 * T)
+    for need in ((True, False, False), (False, True, False), (False, False, True), (False, True, True)):
+        part = race.race_noncausal_backward(qc, kc, vc, gc, state, need=need, tile_tokens=tile)
+        for n, a, b in zip(need, part, full):
+            assert torch.equal(a, b) if n else a is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_infinite_values_stay_where_they_are(race, cuda, dtype):
+    # An infinity in one value column reaches that column's outputs only, as
+    # infinities (the bf16 split of the staged matrix keeps them whole).
+    q, k, v = (x.to(cuda) for x in race.make_inputs(2, 100, 4, 16, 64, seed=9, dtype=dtype))
+    ref = race.race_fused_fwd(q, k, v, causal=False)
+    w = v.clone()
+    w[1, 40, 7] = float("inf")
+    got = race.race_fused_fwd(q, k, w, causal=False)
+    keep = torch.ones_like(ref, dtype=torch.bool)
+    keep[1, :, 7] = False
+    assert torch.equal(got[keep], ref[keep])
+    assert bool((got[1, :, 7] == float("inf")).all())

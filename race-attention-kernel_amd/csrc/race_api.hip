@@ -402,6 +402,12 @@ hipError_t token_map(const void* x, void* out, const MapOperand& op, const Probl
     return launch_token_map(x, out, op, p, Wa, Wb, stream);
 }
 
+// Whether a causal forward without a tiled MFMA specialization runs on the
+// fp32 matrix cores: up to 64 buckets, widths multiples of 4, automatic kernel.
+bool narrow_causal(const Problem& p, int kernel) {
+    return kernel == RACE_KERNEL_AUTO && !mfma_causal_supported(p.S, p.d) && narrow_causal_supported(p.S, p.d);
+}
+
 MapOperand map_operand(const float* m, int64_t stream, int64_t row, int64_t col) {
     MapOperand op;
     op.m = m;
@@ -520,6 +526,15 @@ race_status fwd_impl(const void* probsQ, const void* probsK, const void* V, void
         if (mfma) {
             RACE_TRY(marks->mark(stream));
             return launch_causal_mfma(probsQ, probsK, V, out, records, state, p, stream, marks);
+        }
+        if (narrow_causal(p, p.kernel)) {
+            RACE_TRY(marks->mark(stream));
+            RACE_TRY(launch_nc_sums(probsK, V, records, p, p.S, p.d, stream));
+            RACE_TRY(marks->mark(stream));
+            RACE_TRY(launch_tile_scan(records, state, p, stream));
+            RACE_TRY(marks->mark(stream));
+            RACE_TRY(launch_causal_output_narrow(probsQ, probsK, V, out, records, p, stream));
+            return marks->mark(stream);
         }
         int lds_limit = 0;
         RACE_TRY(max_lds(&lds_limit));
@@ -990,6 +1005,8 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
             RACE_TRY(launch_tile_sums_direct(probsK, V, fwd_ws, p, stream));
         else if (mfma_causal_supported(p.S, p.d))
             RACE_TRY(launch_tile_sums_mfma(probsK, V, fwd_ws, p, stream));
+        else if (narrow_causal(p, kernel))  // the forward's own records, bit for bit
+            RACE_TRY(launch_nc_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         else
             RACE_TRY(launch_tile_outer_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         RACE_TRY(marks->mark(stream));

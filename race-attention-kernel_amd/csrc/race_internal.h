@@ -187,6 +187,13 @@ hipError_t launch_nc_key64(const void* k, const void* v, void* dk, void* dv, con
                            const float* state, const float* dB_ready, const float* dA_ready, const Problem& p,
                            hipStream_t stream);
 
+// ---- causal output pass on the fp32 matrix cores, up to 64 buckets
+// (narrow_causal.hip): shapes without a tiled MFMA specialization, from the
+// scanned records of launch_nc_sums ----
+bool narrow_causal_supported(int S, int d);
+hipError_t launch_causal_output_narrow(const void* q, const void* k, const void* v, void* out, const float* records,
+                                       const Problem& p, hipStream_t stream);
+
 // ---- causal backward (causal_bwd.hip): fp32 vector-ALU kernels ----
 
 // Sub-chunk length (32 or 16) of the causal backward kernels for (S, d) under

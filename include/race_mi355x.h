@@ -355,6 +355,17 @@ race_status race_hash_probs_bwd(const void* x, const float* planes_T, const void
                                 int64_t rows, int32_t head_dim, int32_t num_tables,
                                 int32_t planes_per_table, int32_t dtype, hipStream_t stream);
 
+/* Token rows of several heads to one stream per head: each of the `count` (1
+ * to 3) tensors src[i] [batch][seq_len][heads][head_dim] is copied to dst[i]
+ * [batch * heads][seq_len][head_dim] (the permutes of BatchedACE.forward,
+ * src/race_baseline.py:35-40), in one launch.  `src` and `dst` are host
+ * arrays of device pointers, 16-byte aligned, not overlapping.  Rows are whole
+ * 16-byte chunks: head_dim times the element size a multiple of 16, head_dim
+ * <= 128, batch <= 65535, seq_len * heads <= INT_MAX. */
+race_status race_pack_heads(const void* const* src, void* const* dst, int32_t count, int64_t batch,
+                            int64_t seq_len, int32_t heads, int32_t head_dim, int32_t dtype,
+                            hipStream_t stream);
+
 /* ------------------------------------------------------------------------
  * The causal op with the hashing inside: BatchedACE.forward's hashing and hot
  * span (src/race_baseline.py:41-51) in one op, the reference's fused forward

@@ -55,6 +55,7 @@ EXPORTED_SYMBOLS = (
     "race_causal_bwd_profiled",
     "race_hash_probs",
     "race_hash_probs_bwd",
+    "race_pack_heads",
     "race_hashed_fwd_workspace_bytes",
     "race_hashed_fwd",
     "race_hashed_fwd_profiled",

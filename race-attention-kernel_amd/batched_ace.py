@@ -1,15 +1,17 @@
 """Drop-in BatchedACE (src/race_baseline.py:21-52) running the op on MI355X.
 
-Same constructor and forward signature as the reference module.  The
-permutes of lines 35-40 and 52 stay torch ops.  For the causal module the
-hashing of lines 41-44 (shared hash planes, tanh, corner softmax) and the hot
-span of lines 45-51 run as one op, race_fused_fwd_hashed, whose kernels hash
-the Q and K rows themselves (the reference's fused forward,
-src/race_fused_fwd.cu:80-146), so the bucket probabilities never reach
-memory.  The non-causal module (and a causal one whose L, K, d_k the hashed
-kernels do not take) runs the race_hash_probs kernel and race_fused_fwd.
-Gradients reach Khf, Qhf and Vhf on both paths, as through the reference's
-torch composition; planes_T is a buffer there and here.
+Same constructor and forward signature as the reference module.  The whole
+forward is one op, ModuleRaceFunction: the permutes of lines 35-40 are one
+copy kernel for the three inputs, and the output permute of line 52 is a view.
+For the causal module the hashing of lines 41-44 (shared hash planes, tanh,
+corner softmax) and the hot span of lines 45-51 run in the same kernels, which
+hash the Q and K rows themselves (the reference's fused forward,
+src/race_fused_fwd.cu:80-146), so the bucket probabilities never reach memory.
+The non-causal module runs the hashing kernels and the non-causal op.  A
+causal module whose L, K, d_k the hashed kernels do not take, and a subclass
+with bucket_probs of its own, go through the separate ops.  Gradients reach
+Khf, Qhf and Vhf on every path, as through the reference's torch composition;
+planes_T is a buffer there and here.
 """
 from __future__ import annotations
 
@@ -18,7 +20,8 @@ import itertools
 import torch
 from torch import nn
 
-from .ops import hashed_supported, race_fused_fwd, race_fused_fwd_hashed, race_hash_probs
+from .ops import (ModuleRaceFunction, hashed_supported, race_fused_fwd, race_fused_fwd_hashed,
+                  race_hash_probs)
 
 
 class BatchedACE(nn.Module):
@@ -40,10 +43,14 @@ class BatchedACE(nn.Module):
     def forward(self, Khf, Vhf, Qhf):
         M, B, T, H, dk = Khf.shape
         N = M * B * H
+        hashed = self.causal and hashed_supported(self.L, self.K, dk)
+        own = getattr(self.bucket_probs, "__func__", None) is not BatchedACE.bucket_probs
+        if not own and (hashed or not self.causal):
+            return ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal))
         Kh2 = Khf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
         Qh2 = Qhf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
         V2 = Vhf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
-        if self.causal and hashed_supported(self.L, self.K, dk):
+        if hashed:
             planes = self.planes_T.t().contiguous().float()  # [L*K, d_k]
             out2 = race_fused_fwd_hashed(Kh2, Qh2, V2, planes, self.L)
         else:

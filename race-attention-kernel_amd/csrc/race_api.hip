@@ -1348,6 +1348,24 @@ race_status race_hash_probs_bwd(const void* x, const float* planes_T, const void
 
 }  // extern "C"
 
+extern "C" {
+
+race_status race_pack_heads(const void* const* src, void* const* dst, int32_t count, int64_t batch, int64_t seq_len,
+                            int32_t heads, int32_t head_dim, int32_t dtype, hipStream_t stream) {
+    if (!src || !dst || count < 1 || count > 3) return RACE_ERROR_INVALID_VALUE;
+    if (dtype != RACE_F32 && dtype != RACE_BF16) return RACE_ERROR_INVALID_VALUE;
+    if (batch < 0 || batch > kMaxStreams || seq_len < 0 || heads < 1 || head_dim < 1 || head_dim > 128)
+        return RACE_ERROR_INVALID_VALUE;
+    const int row_bytes = head_dim * (dtype == RACE_BF16 ? 2 : 4);
+    if (row_bytes % 16 != 0 || seq_len > int64_t(INT_MAX) / heads) return RACE_ERROR_INVALID_VALUE;
+    if (batch == 0 || seq_len == 0) return RACE_SUCCESS;
+    for (int i = 0; i < count; ++i)
+        if (!src[i] || !dst[i] || !aligned16(src[i]) || !aligned16(dst[i])) return RACE_ERROR_INVALID_VALUE;
+    return launch_pack_heads(src, dst, count, batch, seq_len, heads, row_bytes, stream);
+}
+
+}  // extern "C"
+
 // ---------------------------------------------------------------------------
 // The causal op with the hashing inside (hashed_causal.hip): the fused
 // forward of src/race_fused_fwd.cu:150-171, race_fused_fwd(K, Q, V, planes, L).

@@ -372,6 +372,10 @@ bool hash_rows_supported(const void* x, const void* probs, const void* dx, int d
 hipError_t launch_hash_rows(const void* x, const float* planes_T, const void* dprobs, void* out, int64_t rows,
                             int dk, int L, int K, int dtype, hipStream_t stream);
 
+// ---- [B][T][H] rows to [B * H][T] rows (pack_heads.hip) ----
+hipError_t launch_pack_heads(const void* const* src, void* const* dst, int count, int64_t batch, int64_t T, int H,
+                             int row_bytes, hipStream_t stream);
+
 // ---- Algorithm 1 with the hashing inside (alg1.hip): bf16 q, k, v, out ----
 struct Alg1Args {
     const void* q;

@@ -15,6 +15,10 @@
 //   hashed_forward(K, Q, V, planes, L, tile_tokens=0, want_records=False, want_state=False)
 //       -> (out, records or None, state or None, tile_tokens): the causal op
 //       with the hashing inside (race_hashed_fwd)
+//   module_forward(K, V, Q, planes_T, L, planes_per_table, causal, needs)
+//       -> (out, saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
+//   module_backward(grad_out, saved, L, planes_per_table, causal, tile_tokens,
+//       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None
 //   hashed_supported(L, K, d) -> bool
 //   select_tile_tokens(N, T, L, R, d, bf16, causal, tile_tokens=0, kernel=0) -> int
 //   shape_supported(L, R, d) -> (supported, has_mfma)
@@ -437,6 +441,47 @@ at::Tensor hash_probs_backward(const at::Tensor& x, const at::Tensor& planes_T,
     return dx;
 }
 
+// [M, B, T, H, d] rows as one stream per head, [M * B * H, T, d] (the permutes
+// of src/race_baseline.py:35-40): one launch for every tensor that is dense,
+// 16-byte aligned, of the first one's shape and dtype and of whole 16-byte
+// rows; the others (and a single head or token, where the permuted view is
+// dense as it stands) through torch.
+std::vector<at::Tensor> streams_of(const std::vector<at::Tensor>& xs) {
+    const at::Tensor& x0 = xs[0];
+    const int64_t es = x0.element_size();
+    auto direct = [&](const at::Tensor& x) {
+        return x.is_cuda() && x.device() == x0.device() && x.scalar_type() == x0.scalar_type() &&
+               (x.scalar_type() == at::kFloat || x.scalar_type() == at::kBFloat16) && x.sizes() == x0.sizes() &&
+               x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    };
+    const int64_t T = x0.size(2), H = x0.size(3), d = x0.size(4);
+    const bool shape_ok = x0.numel() > 0 && H > 1 && T > 1 && d <= 128 && d * es % 16 == 0 &&
+                          x0.size(0) * x0.size(1) <= 65535 && T <= INT32_MAX / H;
+    std::vector<at::Tensor> out;
+    std::vector<const void*> src;
+    std::vector<void*> dst;
+    for (const at::Tensor& x : xs) {
+        if (shape_ok && direct(x)) {
+            out.push_back(at::empty({x0.size(0) * x0.size(1) * H, T, d}, x.options()));
+            src.push_back(x.data_ptr());
+            dst.push_back(out.back().data_ptr());
+        } else {
+            at::Tensor p = x.permute({0, 1, 3, 2, 4}).contiguous();
+            if (reinterpret_cast<uintptr_t>(p.data_ptr()) % 16 != 0) p = p.clone();
+            out.push_back(p.view({p.size(0) * p.size(1) * p.size(2), p.size(3), p.size(4)}));
+        }
+    }
+    if (!src.empty()) {
+        const c10::DeviceGuard guard(x0.device());
+        const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+        check_status(race_pack_heads(src.data(), dst.data(), static_cast<int32_t>(src.size()),
+                                     x0.size(0) * x0.size(1), T, static_cast<int32_t>(H), static_cast<int32_t>(d),
+                                     x0.scalar_type() == at::kBFloat16 ? RACE_BF16 : RACE_F32, stream),
+                     "race_pack_heads");
+    }
+    return out;
+}
+
 // The hashed causal forward's arguments: K, Q, V token rows [N, T, d] of one
 // dtype, planes [L * Kp, d] float32 (the reference's race_fused_fwd(K, Q, V,
 // planes, L), src/race_fused_fwd.cu:150-171).  Returns the shape and Kp.
@@ -527,6 +572,60 @@ int64_t select_tile_tokens(int64_t N, int64_t T, int64_t L, int64_t R, int64_t d
     int32_t tile = 0;
     check_status(race_select_tile_tokens(&sh, causal, &opts, &tile), "race_select_tile_tokens");
     return tile;
+}
+
+// BatchedACE.forward (src/race_baseline.py:34-52) for K, V, Q [M, B, T, H, d]:
+// the heads' rows as streams, the hashing, and the op (causal: with the
+// hashing inside).  Returns the output [M, B, T, H, d] (a permuted view, as
+// the module's own), and with `needs` what module_backward reads: (K, Q, V
+// rows, planes, tile records) and the records' tile length, or (K, Q, V rows,
+// planes_T, probsK, probsQ, state).
+std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at::Tensor& K, const at::Tensor& V,
+                                                                        const at::Tensor& Q,
+                                                                        const at::Tensor& planes_T, int64_t L,
+                                                                        int64_t Kp, bool causal, bool needs) {
+    const int64_t M = K.size(0), B = K.size(1), T = K.size(2), H = K.size(3), d = K.size(4), N = M * B * H;
+    std::vector<at::Tensor> rows = streams_of({K, Q, V});
+    for (at::Tensor& r : rows) r = r.view({N, T, d});
+    at::Tensor out;
+    std::vector<at::Tensor> saved;
+    int64_t tile = 0;
+    if (causal) {
+        const at::Tensor planes = planes_T.t().contiguous().to(at::kFloat);
+        auto r = hashed_forward(rows[0], rows[1], rows[2], planes, L, 0, needs, false);
+        out = std::get<0>(r);
+        if (needs) saved = {rows[0], rows[1], rows[2], planes, *std::get<1>(r)};
+        tile = std::get<3>(r);
+    } else {
+        const at::Tensor pT = planes_T.to(at::kFloat).contiguous();
+        const at::Tensor pk = hash_probs(rows[0], pT, L, Kp), pq = hash_probs(rows[1], pT, L, Kp);
+        auto r = forward(pq, pk, rows[2], false, 0, RACE_KERNEL_AUTO, needs);
+        out = std::get<0>(r);
+        if (needs) saved = {rows[0], rows[1], rows[2], pT, pk, pq, *std::get<1>(r)};
+    }
+    return {out.view({M, B, H, T, d}).permute({0, 1, 3, 2, 4}), saved, tile};
+}
+
+// Gradients of module_forward's rows [N, T, d] (None where not asked for) for
+// the upstream gradient [M, B, T, H, d] of the output.
+std::tuple<c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>> module_backward(
+    const at::Tensor& grad_out, const std::vector<at::Tensor>& saved, int64_t L, int64_t Kp, bool causal, int64_t tile,
+    bool need_k, bool need_v, bool need_q) {
+    const at::Tensor &K = saved[0], &Q = saved[1], &V = saved[2];
+    const at::Tensor g = streams_of({grad_out.to(V.scalar_type())})[0].view(V.sizes());
+    c10::optional<at::Tensor> dq, dk, dv;
+    at::Tensor pT;
+    if (causal) {
+        pT = saved[3].t().contiguous();
+        const at::Tensor pk = hash_probs(K, pT, L, Kp), pq = hash_probs(Q, pT, L, Kp);
+        std::tie(dq, dk, dv) = causal_backward(pq, pk, V, g, need_q, need_k, need_v, tile, RACE_KERNEL_AUTO, saved[4]);
+    } else {
+        pT = saved[3];
+        std::tie(dq, dk, dv) = noncausal_backward(saved[5], saved[4], V, g, saved[6], need_q, need_k, need_v, 0);
+    }
+    if (dk) dk = hash_probs_backward(K, pT, *dk, L, Kp);
+    if (dq) dq = hash_probs_backward(Q, pT, *dq, L, Kp);
+    return {dk, dv, dq};
 }
 
 std::tuple<bool, bool> shape_supported(int64_t L, int64_t R, int64_t d) {
@@ -776,6 +875,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "-> (out, records or None, state or None, tile length)",
           py::arg("K"), py::arg("Q"), py::arg("V"), py::arg("planes"), py::arg("L"),
           py::arg("tile_tokens") = 0, py::arg("want_records") = false, py::arg("want_state") = false);
+    m.def("module_forward", &module_forward, "BatchedACE.forward -> (out, saved, tile_tokens)", py::arg("K"),
+          py::arg("V"), py::arg("Q"), py::arg("planes_T"), py::arg("L"), py::arg("planes_per_table"),
+          py::arg("causal"), py::arg("needs"));
+    m.def("module_backward", &module_backward, "Gradients of module_forward's rows -> (dK, dV, dQ)",
+          py::arg("grad_out"), py::arg("saved"), py::arg("L"), py::arg("planes_per_table"), py::arg("causal"),
+          py::arg("tile_tokens"), py::arg("need_k"), py::arg("need_v"), py::arg("need_q"));
     m.def("hashed_supported", &hashed_supported,
           "Whether the hashed causal forward has kernels for (L, K, d)", py::arg("L"), py::arg("K"),
           py::arg("d"));

@@ -248,6 +248,38 @@ def race_fused_fwd_hashed(K: torch.Tensor, Q: torch.Tensor, V: torch.Tensor, pla
                                     int(tile_tokens))
 
 
+class ModuleRaceFunction(torch.autograd.Function):
+    """BatchedACE.forward as one op: heads to streams, hashing and the op, and
+    their gradients, each direction one call into the binding.
+
+    What it saves is what the separate ops save: copies of the rows (so the
+    inputs may change after the forward), the planes, and the forward's tile
+    records (causal) or the probabilities and the state."""
+
+    @staticmethod
+    def forward(ctx, Khf, Vhf, Qhf, planes_T, L, K, causal):
+        needs = any(ctx.needs_input_grad[:3])
+        out, saved, tile = _lib.ext().module_forward(Khf, Vhf, Qhf, planes_T, L, K, causal, needs)
+        if needs:
+            ctx.save_for_backward(*saved)
+            ctx.args = (L, K, causal, tile)
+            ctx.shapes = (Khf.shape, Vhf.shape, Qhf.shape)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_out):
+        L, K, causal, tile = ctx.args
+        grads = _lib.ext().module_backward(grad_out, ctx.saved_tensors, L, K, causal, tile,
+                                           *ctx.needs_input_grad[:3])
+
+        def heads(g, shape):
+            M, B, T, H, d = shape
+            return None if g is None else g.view(M, B, H, T, d).permute(0, 1, 3, 2, 4)
+
+        return (*(heads(g, s) for g, s in zip(grads, ctx.shapes)), None, None, None, None)
+
+
 def hashed_supported(L: int, K: int, d: int) -> bool:
     """Whether race_fused_fwd_hashed has kernels for L tables of 2^K buckets, width d."""
     return bool(_lib.ext().hashed_supported(int(L), int(K), int(d)))

@@ -192,8 +192,14 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     constexpr bool kQStage = G::kQStage;
     constexpr int kQChunks = C * QT::kChunks;
     constexpr int kQPer = (kQChunks + G::kT - 1) / G::kT;
-    constexpr int kStoreP = std::is_same<TIn, float>::value ? kOutWgStorePolicyF32 : kOutStorePolicy;
-    constexpr int kQP = std::is_same<TIn, float>::value ? kOutQPolicyF32 : kOutQPolicy;
+    // S = d = 64: Q and the output go past the caches, which hold the K and V
+    // rows the tile sums left for this pass (cache_kept_rows).  bf16, N = 8, T =
+    // 131072: 97 us, 89 with Q and 84 with both.  The other bf16 shapes, whose
+    // tile sums leave nothing, keep the default (S = 256, d = 128 ran 997 -> 1015
+    // us with nontemporal stores).
+    constexpr bool kPast = S == 64 && D == 64;
+    constexpr int kStoreP = std::is_same<TIn, float>::value ? kOutWgStorePolicyF32 : kPast ? kPolicyStream : kOutStorePolicy;
+    constexpr int kQP = std::is_same<TIn, float>::value ? kOutQPolicyF32 : kPast ? kPolicyStream : kOutQPolicy;
     // Sub-chunks of operands in flight in registers ahead of the one in LDS.
     constexpr int kDepth = (std::is_same<TIn, float>::value && S == 64 && D == 64) ? RACE_OUT_F32_DEPTH : 1;
 

@@ -13,8 +13,9 @@
 //
 // tile_sums_direct_kernel: per-tile totals B_tile = K^T V and A_tile =
 // colsum(K) (the K1 of the causal decomposition, src/causal_v2/kernels/
-// race_causal_fwd.h:23-27), one wave per tile; tile_sums_quad_kernel: the
-// same for fp32 S = d = 64 with four waves per tile.
+// race_causal_fwd.h:23-27), one wave per tile, for (S, d) = (64, 128) and (128,
+// 64); tile_sums_quad_kernel: the same for fp32 S = d = 64 with four waves per
+// tile (bf16 there: launch_tile_sums_b16, noncausal_mfma.hip).
 #include "mfma_common.h"
 
 namespace race {
@@ -23,18 +24,6 @@ namespace {
 using namespace mfma;
 
 constexpr int kDirC = 32;  // tokens per sub-chunk
-// tile_sums_quad_kernel reads the first RACE_SUMS_F32_ALLOC_EIGHTHS eighths
-// of each tile (the part the output pass reads first, and K1 last) with the
-// cache-allocating policy, the rest `nt`: what the output pass reaches last
-// would have left the memory-side cache by then.  Measured at cfg2 (20 steps
-// after the settling phase, one box): 6/8 3795 M tokens/s, 8/8 3688, 4/8 3745,
-// 2/8 3705 with the same inputs every step; 3476, 3465, 3478, 3442 with two
-// input sets alternating.  On another box, three alternating runs each: 6/8
-// 3810-3843, 5/8 3763-3791, 7/8 3742-3770.
-#ifndef RACE_SUMS_F32_ALLOC_EIGHTHS
-#define RACE_SUMS_F32_ALLOC_EIGHTHS 6
-#endif
-
 // Eight floats (permuted-k order) to bf16 hi/lo fragments.
 template <bool kSplit>
 __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
@@ -191,7 +180,7 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_direct_kernel(
 // sub-chunk pairs (64 tokens) are dealt to the four waves round-robin from
 // the last pair down: at each step the workgroup reads the 256 tokens below
 // the previous step's, so it walks the tile from its end to its start, with
-// cache-allocating loads (kSumsF32LoadPolicy).  The start of every tile is
+// cache-allocating loads for its first `kept` rows (cache_kept_rows).  The start of every tile is
 // then what the 256 MB memory-side cache holds most recently when the output
 // pass, which walks each tile from its start, begins.  The four partial sums
 // meet in LDS and are added in wave order, so the record is the same bit for
@@ -199,7 +188,7 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_direct_kernel(
 template <int S, int D>
 __global__ __launch_bounds__(kThreads, 2) void tile_sums_quad_kernel(
     const float* __restrict__ k, const float* __restrict__ v, float* __restrict__ records, int64_t T,
-    int tile, int64_t tiles, int64_t rec) {
+    int tile, int64_t tiles, int64_t rec, int kept) {
     static_assert(S == 64 && D == 64, "one 64 x 64 block per wave");
     constexpr int C = kDirC, LP = kSumsF32LoadPolicy;
     constexpr int kPart = S * D + S;  // floats of one wave's partial record in LDS
@@ -250,7 +239,7 @@ __global__ __launch_bounds__(kThreads, 2) void tile_sums_quad_kernel(
     int p = pairs - 1 - w;
     const int first = p >= 0 ? 2 * C * p : rows;
     // Pairs from `pcut` up are read `nt`, the rest with the allocating policy.
-    const int pcut = int((int64_t(pairs) * RACE_SUMS_F32_ALLOC_EIGHTHS + 7) / 8);
+    const int pcut = min(pairs, (kept + 2 * C - 1) / (2 * C));
     const int cut = 2 * C * pcut;
     DRows<float, S, LP> k0, k1;
     DRows<float, D, LP> v0, v1;
@@ -534,15 +523,24 @@ bool direct_sums_supported(int S, int d) {
     return (S == 64 && (d == 64 || d == 128)) || (S == 128 && d == 64);
 }
 
+int cache_kept_rows(const Problem& p) {
+    constexpr int64_t kBytes = int64_t(3) << 26;  // 201 MB of the 256 MB memory-side cache
+    const int64_t all = p.N * p.T * (p.S + p.d) * (p.dtype == RACE_BF16 ? 2 : 4);
+    const int64_t most = int64_t(p.tile) * 3 / 4;
+    return all > 0 && p.tile * kBytes / all < most ? int(p.tile * kBytes / all) : int(most);
+}
+
 hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records, const Problem& p,
                                    hipStream_t stream) {
     if (p.tile % (2 * kDirC) != 0) return hipErrorInvalidValue;
     if (p.dtype == RACE_F32 && p.S == 64 && p.d == 64) {
         constexpr size_t kLds = 4 * (64 * 64 + 64) * sizeof(float);
         tile_sums_quad_kernel<64, 64><<<dim3(unsigned(p.tiles), unsigned(p.N)), kThreads, kLds, stream>>>(
-            static_cast<const float*>(k), static_cast<const float*>(v), records, p.T, p.tile, p.tiles, p.rec);
+            static_cast<const float*>(k), static_cast<const float*>(v), records, p.T, p.tile, p.tiles, p.rec,
+            cache_kept_rows(p));
         return hipGetLastError();
     }
+    if (p.dtype == RACE_BF16 && p.S == 64 && p.d == 64) return launch_tile_sums_b16(k, v, records, p, stream);
     const int64_t total = p.N * p.tiles;
     const dim3 grid(unsigned((total + 3) / 4));
 #define RACE_SUMS(TIN, S_, D_, MB)                                                                 \
@@ -550,13 +548,11 @@ hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records,
         static_cast<const TIN*>(k), static_cast<const TIN*>(v), records, p.T, p.tile, p.tiles, p.rec, \
         total)
     if (p.dtype == RACE_F32) {
-        if (p.S == 64 && p.d == 64) RACE_SUMS(float, 64, 64, 1);
-        else if (p.S == 64 && p.d == 128) RACE_SUMS(float, 64, 128, 1);
+        if (p.S == 64 && p.d == 128) RACE_SUMS(float, 64, 128, 1);
         else if (p.S == 128 && p.d == 64) RACE_SUMS(float, 128, 64, 1);
         else return hipErrorInvalidValue;
     } else {
-        if (p.S == 64 && p.d == 64) RACE_SUMS(bf16_t, 64, 64, 1);
-        else if (p.S == 64 && p.d == 128) RACE_SUMS(bf16_t, 64, 128, 1);
+        if (p.S == 64 && p.d == 128) RACE_SUMS(bf16_t, 64, 128, 1);
         else if (p.S == 128 && p.d == 64) RACE_SUMS(bf16_t, 128, 64, 1);
         else return hipErrorInvalidValue;
     }

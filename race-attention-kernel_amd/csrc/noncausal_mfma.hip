@@ -58,9 +58,6 @@ constexpr int kOutside = 0x7ffffff0;  // past any buffer view
 // contraction of a bf16 one.
 template <typename TIn>
 constexpr int kStep = sizeof(TIn) == 4 ? 16 : 32;
-#ifndef kMapWaves
-#define kMapWaves 8
-#endif
 constexpr int kNcStorePolicy = 2;  // nontemporal: the results are not read again here
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
@@ -74,13 +71,14 @@ struct Vec {
     using Raw = std::conditional_t<kBytes == 16, uint4, std::conditional_t<kBytes == 8, uint2, uint32_t>>;
     static_assert(kBytes >= 4, "whole words");
     Raw v;
+    template <int P = mfma::kPolicyDefault>
     __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int off) {
         if constexpr (kBytes == 16)
-            v = mfma::buf_load16<0>(r, off);
+            v = mfma::buf_load16<P>(r, off);
         else if constexpr (kBytes == 8)
-            v = mfma::buf_load8<0>(r, off);
+            v = mfma::buf_load8<P>(r, off);
         else
-            v = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+            v = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, P);
     }
     __device__ __forceinline__ uint32_t word(int i) const {
         if constexpr (kBytes == 16)
@@ -223,10 +221,13 @@ struct Outer {
 // One workgroup per (chunk of tokens, stream, block of R).  Wave w takes the
 // steps w, w + 4, .. of the chunk.  The operand vectors of the next step are
 // loaded before the current step's products.
-template <typename TIn, int EA, int EB>
+// kEndFirst (the causal tile sums, whose tiles the output pass then walks from
+// their start): the steps go from the chunk's end to its start, past the
+// caches except for the first `kept` rows (cache_kept_rows), which come last.
+template <typename TIn, int EA, int EB, bool kEndFirst>
 __global__ __launch_bounds__(kThreads, 3) void nc_sums_kernel(
     const TIn* __restrict__ x, const TIn* __restrict__ y, float* __restrict__ records, int64_t T, int chunk,
-    int64_t chunks, int64_t rec, int Wa, int Wb, int bblocks) {
+    int64_t chunks, int64_t rec, int Wa, int Wb, int bblocks, int kept) {
     extern __shared__ __align__(16) float smem[];
     constexpr int es = int(sizeof(TIn)), kTok = kStep<TIn>, kLoads = kTok / 4;
     const int lane = threadIdx.x & 63, g = lane >> 4, lr = lane & 15;
@@ -240,23 +241,42 @@ __global__ __launch_bounds__(kThreads, 3) void nc_sums_kernel(
     const int ca = a0 + EA * lr, cb = b0 + EB * lr;
     Vec<TIn, EA> xv[kLoads];
     Vec<TIn, EB> yv[kLoads];
-    auto load = [&](int r0) {
+    auto load = [&](auto pol, int r0) {
+        constexpr int P = decltype(pol)::value;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int row = r0 + 4 * i + g;
-            xv[i].load(xr, ca < Wa ? (row * Wa + ca) * es : kOutside);
-            yv[i].load(yr, cb < Wb ? (row * Wb + cb) * es : kOutside);
+            xv[i].template load<P>(xr, ca < Wa ? (row * Wa + ca) * es : kOutside);
+            yv[i].template load<P>(yr, cb < Wb ? (row * Wb + cb) * es : kOutside);
         }
     };
+    using Alloc = std::integral_constant<int, mfma::kPolicyDefault>;
+    using Stream = std::integral_constant<int, mfma::kPolicyStream>;
     Outer<EA, EB> o;
     o.clear();
-    load(kTok * w);
-#pragma unroll 2
-    for (int r0 = kTok * w; r0 < rows; r0 += kTok * kWaves) {
+    // The products of the rows held, the next step's rows loaded meanwhile
+    // (past either end of the chunk: zeros, never used).
+    auto step = [&](auto pol, int next) {
         const Columns<TIn, EA> xc(xv);
         const Columns<TIn, EB> yc(yv);
-        load(r0 + kTok * kWaves);  // past the chunk: zeros
+        load(pol, next);
         o.template add<true>(xc, yc);
+    };
+    constexpr int kAll = kTok * kWaves;
+    if constexpr (kEndFirst) {
+        const int cut = (kept + kAll - 1) / kAll * kAll;
+        int r0 = (rows - 1) / kAll * kAll + kTok * w;
+        if (r0 < cut)
+            load(Alloc{}, r0);
+        else
+            load(Stream{}, r0);
+        for (; r0 - kAll >= cut; r0 -= kAll) step(Stream{}, r0 - kAll);
+#pragma unroll 2
+        for (; r0 >= 0; r0 -= kAll) step(Alloc{}, r0 >= kAll ? r0 - kAll : rows);
+    } else {
+        load(Alloc{}, kTok * w);
+#pragma unroll 2
+        for (int r0 = kTok * w; r0 < rows; r0 += kAll) step(Alloc{}, r0 + kAll);
     }
     o.combine(smem, records + (n * chunks + ci) * rec, Wa, Wb, a0, b0, b0 == 0, w, g, lr);
 }
@@ -800,13 +820,14 @@ int map_wg_tokens(const Problem& p, int slices) {
     return int(((p.T + per - 1) / per + 15) / 16 * 16);
 }
 
-template <typename TIn, int EA, int EB>
+template <typename TIn, int EA, int EB, bool kEndFirst = false>
 hipError_t launch_sums_e(const void* x, const void* y, float* records, const Problem& p, int Wa, int Wb,
                          hipStream_t stream) {
     const int ab = (Wa + 16 * EA - 1) / (16 * EA), bb = (Wb + 16 * EB - 1) / (16 * EB);
     const dim3 grid(unsigned(p.tiles), unsigned(p.N), unsigned(ab * bb));
-    nc_sums_kernel<TIn, EA, EB><<<grid, kThreads, Outer<EA, EB>::kLdsFloats * sizeof(float), stream>>>(
-        static_cast<const TIn*>(x), static_cast<const TIn*>(y), records, p.T, p.tile, p.tiles, p.rec, Wa, Wb, bb);
+    nc_sums_kernel<TIn, EA, EB, kEndFirst><<<grid, kThreads, Outer<EA, EB>::kLdsFloats * sizeof(float), stream>>>(
+        static_cast<const TIn*>(x), static_cast<const TIn*>(y), records, p.T, p.tile, p.tiles, p.rec, Wa, Wb, bb,
+        kEndFirst ? cache_kept_rows(p) : 0);
     return hipGetLastError();
 }
 
@@ -908,6 +929,11 @@ hipError_t launch_nc_sums(const void* x, const void* y, float* records, const Pr
                           hipStream_t stream) {
     if (p.dtype == RACE_BF16) return launch_sums_t<bf16_t>(x, y, records, p, Wa, Wb, stream);
     return launch_sums_t<float>(x, y, records, p, Wa, Wb, stream);
+}
+
+hipError_t launch_tile_sums_b16(const void* k, const void* v, float* records, const Problem& p, hipStream_t stream) {
+    if (p.S != 64 || p.d != 64 || p.dtype != RACE_BF16) return hipErrorInvalidValue;
+    return launch_sums_e<bf16_t, 4, 4, true>(k, v, records, p, 64, 64, stream);
 }
 
 hipError_t launch_nc_map(const void* x, void* out, const MapOperand& op, const Problem& p, int Wa, int Wb,

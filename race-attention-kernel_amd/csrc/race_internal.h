@@ -136,6 +136,18 @@ hipError_t launch_bwd_finalize(const float* dE_records, const float* state, floa
 bool direct_sums_supported(int S, int d);
 hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records, const Problem& p,
                                    hipStream_t stream);
+// Rows at the start of every tile that the tile sums (S = d = 64), walking the
+// tiles from their ends, read last and with cache-allocating loads, so that
+// the output pass, which starts there, finds them in the memory-side cache:
+// 3/4 of the tile, or as many as 3/4 of that cache holds for all tiles
+// together; what the output pass reaches later would have left it by then and
+// is read past the caches (nontemporal reads stream faster).  Measured, fp32,
+// N = 8, T = 65536 (268 MB of K and V) in eighths of the tile: 6/8 3795 M
+// tokens/s, 8/8 3688, 4/8 3745, 2/8 3705; T = 131072, the sums 85.6 us with 6/8
+// and 80 with 3/8 (the cache's share), the output pass 193 either way.  bf16:
+// T = 131072 169 us (one wave per tile walking forward past the caches, output
+// pass 115) -> 134 (output pass 85); T = 1048576 1160 -> 1144.
+int cache_kept_rows(const Problem& p);
 // Register-direct causal output pass: S = d = 64, bf16.
 bool direct_output_supported(int S, int d, int dtype);
 // Tiles per compute unit the direct output pass wants resident (one wave64 per SIMD).
@@ -179,6 +191,9 @@ hipError_t launch_nc_sums(const void* x, const void* y, float* records, const Pr
                           hipStream_t stream);
 hipError_t launch_nc_map(const void* x, void* out, const MapOperand& op, const Problem& p, int Wa, int Wb,
                          hipStream_t stream);
+// The causal tile sums of bf16 tokens at S = d = 64, each tile walked from its
+// end to its start.
+hipError_t launch_tile_sums_b16(const void* k, const void* v, float* records, const Problem& p, hipStream_t stream);
 // S = d = 64: the query side and the key side (dk or dv may be null; dB_ready
 // and dA_ready past kNcFoldParts tiles per stream).
 hipError_t launch_nc_query64(const void* q, const void* g, void* dq, const float* state, float* records,

@@ -12,7 +12,8 @@
 // for t = 0 .. T-1 in order, starting from init (B [S][d] then A [S] per
 // stream) and leaving the advanced state in `state` (when not null).
 //
-// One workgroup per stream holds that stream's whole state in registers:
+// One workgroup per stream (or per 64 value columns of it, launch_decode_typed)
+// holds that stream's whole state in registers:
 // NW = ceil(S / RPT) waves (at most 16), wave w owning the RPT bucket rows
 // [w RPT, (w+1) RPT) and lane c the value columns c and c + 64.  Each wave
 // reads and writes only its own rows of the state, so `state` may be `init`
@@ -34,6 +35,7 @@ namespace {
 
 constexpr int kDecodeGroup = 8;
 constexpr int kDecodeMaxWaves = 16;
+constexpr int kDecodeSplitStreams = 128;  // two workgroups each: one per CU
 
 template <int RPT, int CPT>
 struct DecodeGeo {
@@ -62,6 +64,7 @@ __global__ __launch_bounds__(64 * kDecodeMaxWaves) void decode_kernel(
     const int64_t n = blockIdx.x;
     const int64_t used = int64_t(S) * d + S;
     const int s0 = w * RPT;
+    const int c0 = 64 * CPT * int(blockIdx.y);  // first value column of the workgroup
 
     // The wave's state rows.  Addresses are clamped into the stream's state so
     // that every load is unconditional (a select on a loaded value compiles
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(64 * kDecodeMaxWaves) void decode_kernel(
             const unsigned keep = s0 + i < S ? ~0u : 0u;
 #pragma unroll
             for (int j = 0; j < CPT; ++j) {
-                const int c = lane + 64 * j < d ? lane + 64 * j : d - 1;
+                const int c = c0 + lane + 64 * j < d ? c0 + lane + 64 * j : d - 1;
                 B[i][j] = __uint_as_float(__float_as_uint(st[int64_t(s) * d + c]) & keep);
             }
         }
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(64 * kDecodeMaxWaves) void decode_kernel(
         }
         for (int idx = tid; idx < kDecodeGroup * G::kDP; idx += nthreads) {
             const int tt = idx / G::kDP, c = idx % G::kDP;
-            vs[idx] = (tt < g && c < d) ? to_f32(v[(row0 + tt) * d + c]) : 0.f;
+            vs[idx] = (tt < g && c0 + c < d) ? to_f32(v[(row0 + tt) * d + c0 + c]) : 0.f;
         }
         __syncthreads();
         for (int tt = 0; tt < g; ++tt) {
@@ -139,10 +142,10 @@ __global__ __launch_bounds__(64 * kDecodeMaxWaves) void decode_kernel(
         __syncthreads();
         for (int idx = tid; idx < g * G::kDP; idx += nthreads) {
             const int tt = idx / G::kDP, c = idx % G::kDP;
-            if (c >= d) continue;
+            if (c0 + c >= d) continue;
             float o = ps[tt * G::kDP + c];
             for (int ww = 1; ww < nw; ++ww) o += ps[(ww * kDecodeGroup + tt) * G::kDP + c];
-            store_val(out + (row0 + tt) * d + c, o);
+            store_val(out + (row0 + tt) * d + c0 + c, o);
         }
         // The next group stages into qs, ks, vs after every wave has passed
         // the barrier above (the last reads of this group's rows) and writes
@@ -157,11 +160,13 @@ __global__ __launch_bounds__(64 * kDecodeMaxWaves) void decode_kernel(
         if (s >= S) break;
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
-            const int c = lane + 64 * j;
+            const int c = c0 + lane + 64 * j;
             if (c < d) st[int64_t(s) * d + c] = B[i][j];
         }
     }
-    // Lane i stores A[s0 + i]: one coalesced store per wave.
+    // Lane i stores A[s0 + i]: one coalesced store per wave, by the workgroup of
+    // the first columns.
+    if (c0 != 0) return;
     float a_mine = A[0];
 #pragma unroll
     for (int i = 1; i < RPT; ++i) a_mine = lane == i ? A[i] : a_mine;
@@ -174,7 +179,8 @@ hipError_t launch_decode_t(const void* q, const void* k, const void* v, void* ou
     const int waves = (p.S + RPT - 1) / RPT;
     if (waves > kDecodeMaxWaves) return hipErrorInvalidValue;
     const size_t lds = size_t(DecodeGeo<RPT, CPT>::kLdsFloats) * sizeof(float);
-    decode_kernel<TIn, RPT, CPT><<<dim3(unsigned(p.N)), dim3(64 * waves), lds, stream>>>(
+    const int blocks = (p.d + 64 * CPT - 1) / (64 * CPT);
+    decode_kernel<TIn, RPT, CPT><<<dim3(unsigned(p.N), unsigned(blocks)), dim3(64 * waves), lds, stream>>>(
         static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
         static_cast<TIn*>(out), init, state, p.T, p.S, p.d);
     return hipGetLastError();
@@ -195,7 +201,14 @@ template <typename TIn>
 hipError_t launch_decode_typed(const void* q, const void* k, const void* v, void* out,
                                const float* init, float* state, const Problem& p,
                                hipStream_t stream) {
-    if (p.d <= 64) return launch_decode_rows<TIn, 1>(q, k, v, out, init, state, p, stream);
+    // Wide values and at most one workgroup per CU (256) that way: a workgroup
+    // per 64 columns of a stream (the same sums per column).  Each forms the
+    // stream's mass for itself, so one must not write it while another may
+    // still read it: not for an in-place step.  Measured, bf16, S = 256, d = 128,
+    // one token: N = 1 6.2 -> 4.9 us, N = 128 8.4 -> 7.3, but N = 200 10.7 -> 12.6;
+    // 16 tokens 22.3 -> 17.8, 25.8 -> 21.6, 28.0 -> 38.9.
+    if (p.d <= 64 || (state != init && p.N <= kDecodeSplitStreams))
+        return launch_decode_rows<TIn, 1>(q, k, v, out, init, state, p, stream);
     return launch_decode_rows<TIn, 2>(q, k, v, out, init, state, p, stream);
 }
 

@@ -41,6 +41,7 @@
 // contract over tokens (K^T, V^T) are read transposed from the same tiles with
 // ds_read_b64_tr_b16 (Plane::frag_tr), two reads per fragment and plane.
 #include "causal_geo.h"
+#include "tile_rows.h"
 
 // fp32 S = d = 64 output pass: two sub-chunks of operands in flight in
 // registers ahead of the one in LDS, at two workgroups per CU (the launch
@@ -165,11 +166,16 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_mfma_kernel(
 //   5. B0 += K^T V                             same c-blocks, all s-blocks
 // NW waves per workgroup (4, or 8 where the carried state would otherwise
 // fill the register file: two waves per SIMD then share the CU's work).
-template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise>
+//
+// kFused (short sequences, short_prefixes): the workgroup first sums the tokens
+// before its tile (quad_sums) into its record, and a workgroup past the last
+// tile sums every token into the state when it is asked for: one launch instead
+// of three.
+template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, bool kFused = false>
 __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v,
-    TIn* __restrict__ out, const float* __restrict__ records, int64_t T, int tile, int64_t tiles,
-    int64_t rec) {
+    TIn* __restrict__ out, float* records, int64_t T, int tile, int64_t tiles,
+    int64_t rec, const float* init, float* state) {
     using G = Geo<TIn, S, D, C, NW, kPrecise>;
     using PS = typename G::PS;
     using PK = typename G::PK;
@@ -206,6 +212,13 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     const int tid = threadIdx.x, l = tid & 63, g = l >> 4, lr = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t n = blockIdx.y, ti = blockIdx.x;
+    if constexpr (kFused) {
+        if (ti == tiles) {
+            quad_sums<TIn>(k + n * T * S, v + n * T * D, int(T), int(T), reinterpret_cast<float*>(lds),
+                           state + n * (S * D + S), init ? init + n * (S * D + S) : nullptr);
+            return;
+        }
+    }
     const int64_t t_begin = ti * tile;
     const int64_t t_end = min(T, t_begin + tile);
     const int rows = int(t_end - t_begin);
@@ -215,7 +228,13 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     const __amdgpu_buffer_rsrc_t or_ = make_rsrc(out + (n * T + t_begin) * D, int64_t(rows) * D * sizeof(TIn));
 
     // Carried state from the tile's exclusive prefix record.
-    const float* rec_p = records + (n * tiles + ti) * rec;
+    float* rec_p = records + (n * tiles + ti) * rec;
+    if constexpr (kFused) {
+        static_assert(S == 64 && D == 64 && NW == 4, "quad_sums");
+        quad_sums<TIn>(k + n * T * S, v + n * T * D, int(t_begin), int(t_begin), reinterpret_cast<float*>(lds), rec_p,
+                       init ? init + n * (S * D + S) : nullptr);
+        __syncthreads();
+    }
     f32x4 b0[NSB][CBW];
 #pragma unroll
     for (int sb = 0; sb < NSB; ++sb)
@@ -457,14 +476,31 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     using GO = Geo<TIn, S, D, C, NW, kPrecise>;
     static_assert(GO::kOutputLds <= 160 * 1024, "gfx950 gives a workgroup at most 160 KB of LDS");
     const dim3 grid(unsigned(p.tiles), unsigned(p.N));
-    hipError_t err = launch_sums_family<TIn, S, D, C, kMinBlocks>(k, v, records, p, stream);
+    hipError_t err = hipSuccess;
+    if constexpr (S == 64 && D == 64) {
+        // One launch; the marks of the three keep their places.  (A state must not
+        // be written over the carried one while other workgroups still read it.)
+        if (short_prefixes(p) && (!state || state != p.init)) {
+            if (marks && ((err = marks->mark(stream)) != hipSuccess || (err = marks->mark(stream)) != hipSuccess))
+                return err;
+            constexpr size_t kQuad = kQuadLdsFloats * sizeof(float);
+            constexpr size_t kLds = size_t(GO::kOutputLds) > kQuad ? size_t(GO::kOutputLds) : kQuad;
+            const dim3 fused(unsigned(p.tiles + (state ? 1 : 0)), unsigned(p.N));
+            causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, true><<<fused, GO::kT, kLds, stream>>>(
+                static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
+                static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, p.init, state);
+            if ((err = hipGetLastError()) != hipSuccess) return err;
+            return marks ? marks->mark(stream) : hipSuccess;
+        }
+    }
+    err = launch_sums_family<TIn, S, D, C, kMinBlocks>(k, v, records, p, stream);
     if (err != hipSuccess) return err;
     if (marks && (err = marks->mark(stream)) != hipSuccess) return err;
     if ((err = launch_tile_scan(records, state, p, stream)) != hipSuccess) return err;
     if (marks && (err = marks->mark(stream)) != hipSuccess) return err;
     causal_output_mfma_kernel<TIn, S, D, C, kMinBlocks, NW, kPrecise><<<grid, GO::kT, GO::kOutputLds, stream>>>(
         static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
-        static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec);
+        static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, nullptr, nullptr);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (marks) return marks->mark(stream);

@@ -16,49 +16,12 @@
 // race_causal_fwd.h:23-27), one wave per tile, for (S, d) = (64, 128) and (128,
 // 64); tile_sums_quad_kernel: the same for fp32 S = d = 64 with four waves per
 // tile (bf16 there: launch_tile_sums_b16, noncausal_mfma.hip).
-#include "mfma_common.h"
+#include "tile_rows.h"
 
 namespace race {
 namespace {
 
 using namespace mfma;
-
-constexpr int kDirC = 32;  // tokens per sub-chunk
-// Eight floats (permuted-k order) to bf16 hi/lo fragments.
-template <bool kSplit>
-__device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
-    uint2 h0, l0, h1, l1;
-    split4<kSplit>(v[0], v[1], v[2], v[3], h0, l0);
-    split4<kSplit>(v[4], v[5], v[6], v[7], h1, l1);
-    hi = __builtin_bit_cast(bf16x8, make_uint4(h0.x, h0.y, h1.x, h1.y));
-    if constexpr (kSplit) lo = __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
-}
-
-// One sub-chunk of a [tokens][W] tensor in the lane layout above.
-template <typename TIn, int W, int P>
-struct DRows {
-    static constexpr int NG = W / 64;
-    f32x4 x[NG][2][4];  // [column group][h][r]: columns 64 gg + 4 lr .. + 3 of row 16 h + 4 g + r
-
-    template <int PP = P>
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int r0, int g, int lr) {
-#pragma unroll
-        for (int gg = 0; gg < NG; ++gg)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    x[gg][h][r] = load_q4<TIn, PP>(
-                        rs, ((r0 + 16 * h + 4 * g + r) * W + 64 * gg + 4 * lr) * int(sizeof(TIn)));
-    }
-    // The 8 rows of column 64 gg + 4 lr + c, in permuted-k order.
-    __device__ __forceinline__ void col(int gg, int c, float (&v)[8]) const {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[4 * h + r] = x[gg][h][r][c];
-    }
-};
 
 __device__ __forceinline__ bool direct_tile(int64_t total_tiles, int64_t tiles, int w, int64_t* n,
                                             int64_t* ti) {
@@ -176,126 +139,23 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_direct_kernel(
 
 // ---------------------------------------------------------------------------
 // K1 for fp32 S = d = 64: one workgroup per tile, so the launch spreads over
-// every CU (one wave per tile left half of them idle at cfg2).  The tile's
-// sub-chunk pairs (64 tokens) are dealt to the four waves round-robin from
-// the last pair down: at each step the workgroup reads the 256 tokens below
-// the previous step's, so it walks the tile from its end to its start, with
-// cache-allocating loads for its first `kept` rows (cache_kept_rows).  The start of every tile is
-// then what the 256 MB memory-side cache holds most recently when the output
-// pass, which walks each tile from its start, begins.  The four partial sums
-// meet in LDS and are added in wave order, so the record is the same bit for
-// bit on every run.
-template <int S, int D>
+// every CU (one wave per tile left half of them idle at cfg2).  The walk from
+// the tile's end to its start leaves its first `kept` rows (cache_kept_rows) in
+// the 256 MB memory-side cache, where the output pass, which walks each tile
+// from its start, begins.
+// kPrefix: the record of tile ti is the sum over every token before it instead
+// (few short tiles: no scan is needed), with the carried state `init` ([N][S d +
+// S]) when it is given.
+template <typename TIn, bool kPrefix>
 __global__ __launch_bounds__(kThreads, 2) void tile_sums_quad_kernel(
-    const float* __restrict__ k, const float* __restrict__ v, float* __restrict__ records, int64_t T,
-    int tile, int64_t tiles, int64_t rec, int kept) {
-    static_assert(S == 64 && D == 64, "one 64 x 64 block per wave");
-    constexpr int C = kDirC, LP = kSumsF32LoadPolicy;
-    constexpr int kPart = S * D + S;  // floats of one wave's partial record in LDS
-    extern __shared__ __align__(16) float part[];  // [4][kPart]
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
+    const TIn* __restrict__ k, const TIn* __restrict__ v, float* __restrict__ records, int64_t T,
+    int tile, int64_t tiles, int64_t rec, int kept, const float* __restrict__ init) {
+    extern __shared__ __align__(16) float part[];
     const int64_t n = blockIdx.y, ti = blockIdx.x;
-    const int64_t t_begin = ti * tile;
-    const int rows = int(min<int64_t>(T, t_begin + tile) - t_begin);
-    const __amdgpu_buffer_rsrc_t kr = make_rsrc(k + (n * T + t_begin) * S, int64_t(rows) * S * 4);
-    const __amdgpu_buffer_rsrc_t vr = make_rsrc(v + (n * T + t_begin) * D, int64_t(rows) * D * 4);
-
-    f32x4 acc[4][4];  // [sb][cb]: B[4 (4 g + r) + sb][4 lr + cb] at element r
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) acc[sb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float asum[4] = {0.f, 0.f, 0.f, 0.f};
-
-    // Consume the sub-chunk held in (kx, vx), then refill them from row
-    // `next` (past the tile the loads read zeros, which are never consumed).
-    auto chunk = [&](auto pol, DRows<float, S, LP>& kx, DRows<float, D, LP>& vx, int next) {
-        constexpr int PP = decltype(pol)::value;
-        bf16x8 vh[4], vl[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) {
-            float e[8];
-            vx.col(0, cb, e);
-            split8<true>(e, vh[cb], vl[cb]);
-        }
-        vx.template load<PP>(vr, next, g, lr);
-#pragma unroll
-        for (int sb = 0; sb < 4; ++sb) {
-            float e[8];
-            kx.col(0, sb, e);
-            asum[sb] += (((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7])));
-            bf16x8 kh, kl;
-            split8<true>(e, kh, kl);
-#pragma unroll
-            for (int cb = 0; cb < 4; ++cb) acc[sb][cb] = mfma3<true>(kh, kl, vh[cb], vl[cb], acc[sb][cb]);
-        }
-        kx.template load<PP>(kr, next, g, lr);
-    };
-
-    // Pair p covers rows 2 C p .. 2 C p + 2 C - 1 (the second half may lie
-    // past the tile and read zeros).  Wave w takes pairs P-1-w, P-5-w, ...
-    const int pairs = (rows + 2 * C - 1) / (2 * C);
-    int p = pairs - 1 - w;
-    const int first = p >= 0 ? 2 * C * p : rows;
-    // Pairs from `pcut` up are read `nt`, the rest with the allocating policy.
-    const int pcut = min(pairs, (kept + 2 * C - 1) / (2 * C));
-    const int cut = 2 * C * pcut;
-    DRows<float, S, LP> k0, k1;
-    DRows<float, D, LP> v0, v1;
-    if (first < cut) {
-        k0.load(kr, first, g, lr);
-        v0.load(vr, first, g, lr);
-        k1.load(kr, first + C, g, lr);
-        v1.load(vr, first + C, g, lr);
-    } else {
-        k0.template load<kPolicyStream>(kr, first, g, lr);
-        v0.template load<kPolicyStream>(vr, first, g, lr);
-        k1.template load<kPolicyStream>(kr, first + C, g, lr);
-        v1.template load<kPolicyStream>(vr, first + C, g, lr);
-    }
-    using Alloc = std::integral_constant<int, LP>;
-    using Stream = std::integral_constant<int, kPolicyStream>;
-    for (; p - 4 >= pcut; p -= 4) {
-        const int nx = 2 * C * (p - 4);
-        chunk(Stream{}, k0, v0, nx);
-        chunk(Stream{}, k1, v1, nx + C);
-    }
-    for (; p >= 0; p -= 4) {
-        const int nx = 2 * C * (p - 4);  // below row 0 (last round): outside the range, zeros
-        chunk(Alloc{}, k0, v0, nx);
-        chunk(Alloc{}, k1, v1, nx + C);
-    }
-
-    // Partial record of wave w: B row 16 g + 4 r + sb, columns 4 lr .. + 3,
-    // then A (the token groups g added in a fixed order).
-    float* mine = part + w * kPart;
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<f32x4*>(mine + (16 * g + 4 * r + sb) * D + 4 * lr) =
-                f32x4{acc[sb][0][r], acc[sb][1][r], acc[sb][2][r], acc[sb][3][r]};
-    {
-        f32x4 a;
-#pragma unroll
-        for (int sb = 0; sb < 4; ++sb) {
-            float x = asum[sb];
-            x = x + __shfl_xor(x, 16);
-            x = x + __shfl_xor(x, 32);
-            a[sb] = x;
-        }
-        if (g == 0) *reinterpret_cast<f32x4*>(mine + S * D + 4 * lr) = a;
-    }
-    __syncthreads();
-    // record = ((part0 + part1) + part2) + part3, 16-byte pieces.
-    float* rp = records + (n * tiles + ti) * rec;
-    for (int i = threadIdx.x; i < kPart / 4; i += kThreads) {
-        f32x4 x = *reinterpret_cast<const f32x4*>(part + 4 * i);
-#pragma unroll
-        for (int j = 1; j < 4; ++j) x += *reinterpret_cast<const f32x4*>(part + j * kPart + 4 * i);
-        *reinterpret_cast<f32x4*>(rp + 4 * i) = x;
-    }
+    const int64_t t_begin = kPrefix ? 0 : ti * tile;
+    const int rows = int(min<int64_t>(T, (kPrefix ? ti : ti + 1) * int64_t(tile)) - t_begin);
+    quad_sums<TIn>(k + (n * T + t_begin) * 64, v + (n * T + t_begin) * 64, rows, kPrefix ? rows : kept, part,
+                   records + (n * tiles + ti) * rec, kPrefix && init ? init + n * (64 * 64 + 64) : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -519,6 +379,24 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void causal_output_direct_ker
 
 }  // namespace
 
+bool short_prefixes(const Problem& p) {
+    return p.S == 64 && p.d == 64 && (p.tiles - 1) * int64_t(p.tile) <= kShortPrefixTokens &&
+           (p.tiles <= 6 || p.N * p.tiles <= 512);
+}
+
+hipError_t launch_prefix_records(const void* k, const void* v, float* records, const Problem& p, hipStream_t stream) {
+    if (!short_prefixes(p)) return hipErrorInvalidValue;
+    const dim3 grid(unsigned(p.tiles), unsigned(p.N));
+    constexpr size_t kLds = kQuadLdsFloats * sizeof(float);
+    if (p.dtype == RACE_BF16)
+        tile_sums_quad_kernel<bf16_t, true><<<grid, kThreads, kLds, stream>>>(
+            static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), records, p.T, p.tile, p.tiles, p.rec, 0, p.init);
+    else
+        tile_sums_quad_kernel<float, true><<<grid, kThreads, kLds, stream>>>(
+            static_cast<const float*>(k), static_cast<const float*>(v), records, p.T, p.tile, p.tiles, p.rec, 0, p.init);
+    return hipGetLastError();
+}
+
 bool direct_sums_supported(int S, int d) {
     return (S == 64 && (d == 64 || d == 128)) || (S == 128 && d == 64);
 }
@@ -534,10 +412,10 @@ hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records,
                                    hipStream_t stream) {
     if (p.tile % (2 * kDirC) != 0) return hipErrorInvalidValue;
     if (p.dtype == RACE_F32 && p.S == 64 && p.d == 64) {
-        constexpr size_t kLds = 4 * (64 * 64 + 64) * sizeof(float);
-        tile_sums_quad_kernel<64, 64><<<dim3(unsigned(p.tiles), unsigned(p.N)), kThreads, kLds, stream>>>(
+        constexpr size_t kLds = kQuadLdsFloats * sizeof(float);
+        tile_sums_quad_kernel<float, false><<<dim3(unsigned(p.tiles), unsigned(p.N)), kThreads, kLds, stream>>>(
             static_cast<const float*>(k), static_cast<const float*>(v), records, p.T, p.tile, p.tiles, p.rec,
-            cache_kept_rows(p));
+            cache_kept_rows(p), nullptr);
         return hipGetLastError();
     }
     if (p.dtype == RACE_BF16 && p.S == 64 && p.d == 64) return launch_tile_sums_b16(k, v, records, p, stream);

@@ -1001,7 +1001,9 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
     RACE_TRY(marks->mark(stream));
     const float* fwd_rec = fwd_records;
     if (!fwd_rec && !whole_streams) {
-        if (direct_sums_supported(p.S, p.d) && p.tile % 64 == 0)
+        if (short_prefixes(p))  // the forward's own records, bit for bit
+            RACE_TRY(launch_prefix_records(probsK, V, fwd_ws, p, stream));
+        else if (direct_sums_supported(p.S, p.d) && p.tile % 64 == 0)
             RACE_TRY(launch_tile_sums_direct(probsK, V, fwd_ws, p, stream));
         else if (mfma_causal_supported(p.S, p.d))
             RACE_TRY(launch_tile_sums_mfma(probsK, V, fwd_ws, p, stream));
@@ -1010,7 +1012,7 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
         else
             RACE_TRY(launch_tile_outer_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         RACE_TRY(marks->mark(stream));
-        RACE_TRY(launch_tile_scan(fwd_ws, nullptr, p, stream));
+        if (!short_prefixes(p)) RACE_TRY(launch_tile_scan(fwd_ws, nullptr, p, stream));
         RACE_TRY(marks->mark(stream));
         fwd_rec = fwd_ws;
     }

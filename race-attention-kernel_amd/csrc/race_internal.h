@@ -148,6 +148,20 @@ hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records,
 // T = 131072 169 us (one wave per tile walking forward past the caches, output
 // pass 115) -> 134 (output pass 85); T = 1048576 1160 -> 1144.
 int cache_kept_rows(const Problem& p);
+// Short sequences at S = d = 64, whose last tile starts within
+// kShortPrefixTokens tokens: every tile's prefix is summed from the first token
+// (short_prefixes), which saves the scan, and in the forward the tile sums'
+// launch too (each output workgroup sums its own).  With more than six tiles
+// only where every workgroup is resident at once (two per CU): the tokens
+// summed again otherwise cost what the launches saved.  Measured, the whole
+// forward, fp32: N = 8, T = 512 13.8 -> 11.6 us, N = 1, T = 64 12.2 -> 7.6, N =
+// 512, T = 512 (one tile) 79 -> 57, N = 128, T = 512 (4 tiles) 29.8 -> 28.5; bf16 N
+// = 64, T = 512 (8 tiles, 512 workgroups) 21.2 -> 15.2, but N = 128 (1024) 26.6 ->
+// 27.3.
+constexpr int64_t kShortPrefixTokens = 512;
+bool short_prefixes(const Problem& p);
+// The exclusive prefix records (from p.init when it is not null), one launch.
+hipError_t launch_prefix_records(const void* k, const void* v, float* records, const Problem& p, hipStream_t stream);
 // Register-direct causal output pass: S = d = 64, bf16.
 bool direct_output_supported(int S, int d, int dtype);
 // Tiles per compute unit the direct output pass wants resident (one wave64 per SIMD).

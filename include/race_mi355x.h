@@ -66,7 +66,9 @@ typedef enum race_dtype {
 } race_dtype;
 
 /* Which kernels run.  AUTO picks the MFMA kernels where a specialization
- * exists for (S, d) and the VALU kernels otherwise.  VALU forces the fp32
+ * exists for (S, d), other matrix-core passes where there are any (the causal
+ * forward up to 64 buckets, the non-causal op) and the VALU kernels
+ * otherwise.  VALU forces the fp32
  * vector-ALU kernels (the reference-shaped path, any supported shape); MFMA
  * forces the matrix-core kernels and fails with RACE_ERROR_INVALID_VALUE if
  * the shape has none.  The MFMA path runs one wave per tile where a tile's

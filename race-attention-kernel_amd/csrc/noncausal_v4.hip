@@ -1,5 +1,6 @@
 // noncausal_v4.hip -- vector-ALU bucket reductions and token maps of the
-// non-causal forward and backward for widths that are multiples of 4.
+// non-causal forward and backward for widths that are multiples of 4, as
+// RACE_KERNEL_VALU selects them (noncausal_mfma.hip otherwise).
 //
 // The non-causal function (analysis/hot-path.md:157-162) and its VJP are two
 // kinds of pass over the tokens:

@@ -170,12 +170,13 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_mfma_kernel(
 // kFused (short sequences, short_prefixes): the workgroup first sums the tokens
 // before its tile (quad_sums) into its record, and a workgroup past the last
 // tile sums every token into the state when it is asked for: one launch instead
-// of three.
+// of three.  Its records are `prefixes`, which it writes; `records` stays a
+// read-only operand of the unfused pass.
 template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, bool kFused = false>
 __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v,
-    TIn* __restrict__ out, float* records, int64_t T, int tile, int64_t tiles,
-    int64_t rec, const float* init, float* state) {
+    TIn* __restrict__ out, const float* __restrict__ records, int64_t T, int tile, int64_t tiles,
+    int64_t rec, float* prefixes, const float* init, float* state) {
     using G = Geo<TIn, S, D, C, NW, kPrecise>;
     using PS = typename G::PS;
     using PK = typename G::PK;
@@ -228,10 +229,11 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     const __amdgpu_buffer_rsrc_t or_ = make_rsrc(out + (n * T + t_begin) * D, int64_t(rows) * D * sizeof(TIn));
 
     // Carried state from the tile's exclusive prefix record.
-    float* rec_p = records + (n * tiles + ti) * rec;
+    const float* rec_p = (kFused ? prefixes : records) + (n * tiles + ti) * rec;
     if constexpr (kFused) {
+        float* own = prefixes + (n * tiles + ti) * rec;
         static_assert(S == 64 && D == 64 && NW == 4, "quad_sums");
-        quad_sums<TIn>(k + n * T * S, v + n * T * D, int(t_begin), int(t_begin), reinterpret_cast<float*>(lds), rec_p,
+        quad_sums<TIn>(k + n * T * S, v + n * T * D, int(t_begin), int(t_begin), reinterpret_cast<float*>(lds), own,
                        init ? init + n * (S * D + S) : nullptr);
         __syncthreads();
     }
@@ -488,7 +490,7 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
             const dim3 fused(unsigned(p.tiles + (state ? 1 : 0)), unsigned(p.N));
             causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, true><<<fused, GO::kT, kLds, stream>>>(
                 static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
-                static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, p.init, state);
+                static_cast<TIn*>(out), nullptr, p.T, p.tile, p.tiles, p.rec, records, p.init, state);
             if ((err = hipGetLastError()) != hipSuccess) return err;
             return marks ? marks->mark(stream) : hipSuccess;
         }
@@ -500,7 +502,7 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     if (marks && (err = marks->mark(stream)) != hipSuccess) return err;
     causal_output_mfma_kernel<TIn, S, D, C, kMinBlocks, NW, kPrecise><<<grid, GO::kT, GO::kOutputLds, stream>>>(
         static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
-        static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, nullptr, nullptr);
+        static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, nullptr, nullptr, nullptr);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (marks) return marks->mark(stream);

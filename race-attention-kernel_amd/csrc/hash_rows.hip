@@ -343,10 +343,14 @@ __global__ __launch_bounds__(kThreads) void hash_rows_bwd_kernel(
                     for (int k = 0; k + 2 < K; ++k)
                         if ((u >> (K - 3 - k)) & 1) pos[k] += q4;
                 }
+                // The slots of a table past L take part in the products below: a
+                // row with an infinity left NaN in them (0 * inf).
+                const bool there = SL::table(b, 4 * g + 2 * t) < L;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const float tk = th[2 * t + k];
-                    dp[2 * t + k] = 2.0f * (pos[k] - s[k] * tot) * (1.0f - tk * tk) * inv_scale;
+                    const float du = 2.0f * (pos[k] - s[k] * tot) * (1.0f - tk * tk) * inv_scale;
+                    dp[2 * t + k] = there ? du : 0.f;
                 }
             }
 #pragma unroll

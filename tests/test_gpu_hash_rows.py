@@ -76,3 +76,30 @@ def test_a_row_only_sees_itself(race, cuda):
     keep[3] = keep[18] = False
     assert torch.equal(got[keep], ref[keep])
     assert bool(got[3].isnan().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk, L, K", [(64, 1, 2), (64, 9, 2), (64, 2, 3), (64, 1, 4), (64, 4, 4), (128, 5, 4),
+                                      (64, 2, 5), (60, 3, 6)])
+def test_gradient_of_rows_with_infinities(race, cuda, dtype, dk, L, K):
+    # A row with one infinity has every plane at tanh(+-inf) = +-1, whose
+    # derivative is zero: its gradient is zero, also where the tables leave
+    # slots of their set empty, and every other row keeps its bits.
+    say("hash rows inf", dtype, dk, L, K)
+    gen = torch.Generator().manual_seed(dk + L + K)
+    x = torch.randn(40, dk, generator=gen).to(dtype).to(cuda)
+    planes_T = torch.randn(dk, L * K, generator=gen).to(cuda)
+    g = torch.randn(40, L, 1 << K, generator=gen).to(dtype).to(cuda)
+    y = x.clone()
+    y[18, 5] = float("inf")
+    y[3, dk - 1] = -float("inf")
+
+    def grad(rows):
+        rows = rows.requires_grad_(True)
+        return torch.autograd.grad(race.race_hash_probs(rows, planes_T, L, K), rows, g)[0]
+
+    ref, got = grad(x), grad(y)
+    assert bool((got[[3, 18]] == 0).all()), got[[3, 18]]
+    keep = torch.ones(40, dtype=torch.bool, device=cuda)
+    keep[[3, 18]] = False
+    assert torch.equal(got[keep], ref[keep])

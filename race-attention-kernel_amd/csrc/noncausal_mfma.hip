@@ -11,7 +11,8 @@
 // bf16 tokens: v_mfma_f32_16x16x32_bf16, sixteen times that rate.  A reduction's
 // products of two bf16 values are exact in its fp32 sums; a map's fp32 matrix
 // is split into three bf16 terms that add up to it exactly (8 bits each,
-// truncated), so its products are the fp32 ones too.
+// truncated), so its products are the fp32 ones too (for finite tokens; those
+// with an infinity or NaN take fp32 products, whole_products).
 // The token rows never go through workgroup-wide LDS staging: a wave loads
 // whole rows into registers and, where the products want the other layout,
 // turns 16 or 32 rows through a piece of LDS of its own, without barriers.
@@ -326,6 +327,22 @@ struct MapRows {
 #pragma unroll
         for (int j = 0; j < kOps; ++j) x[j].v = t[at(lr, 4 * j + g)];
     }
+    // The lanes that hold an infinity or NaN, where the products are of terms:
+    // a zero term times an infinity is NaN, so those tokens need whole_products.
+    __device__ __forceinline__ uint64_t nonfinite() const {
+        if constexpr (kB16) {
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+            u16x2 top = {0, 0};
+#pragma unroll
+            for (int j = 0; j < kOps; ++j)
+#pragma unroll
+                for (int i = 0; i < kUnit / 4; ++i)
+                    top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, x[j].word(i) & 0x7fff7fffu));
+            return __ballot(top[0] >= 0x7f80 || top[1] >= 0x7f80);
+        } else {
+            return 0;
+        }
+    }
     template <int NCB>
     __device__ __forceinline__ void times(const float* __restrict__ m, int lane, f32x4 (&acc)[NCB]) const {
         if constexpr (kB16) {
@@ -417,17 +434,22 @@ struct OutRows {
     static constexpr int kBytes = 16 * kUnits * 4 * int(sizeof(TIn));
     using Raw = std::conditional_t<sizeof(TIn) == 4, u32x4, u32x2>;
     __device__ __forceinline__ static int at(int row, int u) { return row * kUnits + (u ^ (row & (kUnits - 1))); }
-    // Rows row0 .. of the view `o`, row length W; columns c0 .. of it, ncols of them.
+    __device__ __forceinline__ static void put(Raw* __restrict__ t, int cb, const f32x4& y, int g, int lr) {
+        if constexpr (sizeof(TIn) == 4)
+            t[at(lr, 4 * cb + g)] = __builtin_bit_cast(u32x4, y);
+        else
+            t[at(lr, 4 * cb + g)] = u32x2{mfma::pack2(y[0], y[1]), mfma::pack2(y[2], y[3])};
+    }
+    // Rows row0 .. of the view `o`, row length W; columns c0 .. of it, ncols of
+    // them.  `replace` runs with the results in `t`.
+    template <typename Replace>
     __device__ __forceinline__ static void store(Raw* __restrict__ t, const f32x4 (&acc)[NCB], __amdgpu_buffer_rsrc_t o,
-                                                 int row0, int W, int c0, int ncols, int lane, int g, int lr) {
+                                                 int row0, int W, int c0, int ncols, int lane, int g, int lr,
+                                                 Replace replace) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) {
-            if constexpr (sizeof(TIn) == 4)
-                t[at(lr, 4 * cb + g)] = __builtin_bit_cast(u32x4, acc[cb]);
-            else
-                t[at(lr, 4 * cb + g)] = u32x2{mfma::pack2(acc[cb][0], acc[cb][1]), mfma::pack2(acc[cb][2], acc[cb][3])};
-        }
+        for (int cb = 0; cb < NCB; ++cb) put(t, cb, acc[cb], g, lr);
+        replace();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int i = 0; i < NCB; ++i) {
@@ -441,6 +463,40 @@ struct OutRows {
         }
     }
 };
+
+// The results in `t` of the tokens whose lanes are set in `bad` (bf16 rows row0
+// .. of `xr`, row length W; MapRows::nonfinite), replaced by the products with
+// the staged matrix put together again from its terms: fp32 products, as the
+// other tokens' terms add up to.  init(cb, g) gives the values a lane's sums
+// start from.  Operands are read again and nothing is unrolled: rows like these are
+// the exception, and the registers the loop around it holds are not.
+template <typename TIn, int NJ, int NCB, typename Init>
+__device__ __forceinline__ void whole_products(typename OutRows<TIn, NCB>::Raw* __restrict__ t, uint64_t bad,
+                                               __amdgpu_buffer_rsrc_t xr, int row0, int W,
+                                               const float* __restrict__ m, int lane, Init init) {
+    using X = MapRows<TIn, NJ, true>;
+    asm volatile("" : "+v"(lane));  // the addresses below are not kept for the loop either
+    const int g = lane >> 4, lr = lane & 15;
+    const bool mine = ((bad | bad >> 16 | bad >> 32 | bad >> 48) >> lr) & 1;
+    const uint2* mt = reinterpret_cast<const uint2*>(m);
+#pragma unroll 1
+    for (int cb = 0; cb < NCB; ++cb) {
+        f32x4 acc = init(cb, g);
+#pragma unroll 1
+        for (int h = 0; h < 2 * X::kOps; ++h) {  // half operands
+            const int j = h >> 1, c = 32 * j + 8 * g + 4 * (h & 1);
+            Vec<bf16_t, 4> x, t0, t1, t2;
+            x.load(xr, c < W ? ((row0 + lr) * W + c) * int(sizeof(TIn)) : kOutside);
+            const uint2* at = mt + ((j * NCB + cb) * 3 * 64 + lane) * 2 + (h & 1);
+            t0.v = at[0];
+            t1.v = at[128];
+            t2.v = at[256];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = mfma4(t0.get(e) + (t1.get(e) + t2.get(e)), x.get(e), acc);
+        }
+        if (mine) OutRows<TIn, NCB>::put(t, cb, acc, g, lr);
+    }
+}
 
 // Columns c0 .. c0 + 16 NCB - 1 of the map operand's matrix in operand order,
 // zero past Wa rows and `ncols` columns; the workgroups of a stream's first
@@ -569,14 +625,18 @@ __global__ __launch_bounds__(64 * NW) void nc_map_kernel(const TIn* __restrict__
     X next;
     load(next, 16 * w);
     stage_operand<64 * NW, NJ, NCB, kB16>(smem, op, n, Wa, c0, ncols, blk == 0, blockIdx.y == 0);
-    f32x4 bias[NCB];
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb)
+    auto bias_of = [&](int cb, int g) {
+        f32x4 b;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int c = 16 * cb + 4 * g + r;
-            bias[cb][r] = op.bias && c < ncols ? op.bias[n * op.bias_stream + c0 + c] : 0.f;
+            b[r] = op.bias && c < ncols ? op.bias[n * op.bias_stream + c0 + c] : 0.f;
         }
+        return b;
+    };
+    f32x4 bias[NCB];
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) bias[cb] = bias_of(cb, g);
     __syncthreads();
     for (int r0 = 16 * w; r0 < rows; r0 += 16 * NW) {
         X cur = next;
@@ -585,8 +645,14 @@ __global__ __launch_bounds__(64 * NW) void nc_map_kernel(const TIn* __restrict__
         f32x4 acc[NCB];
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) acc[cb] = bias[cb];
+        const uint64_t bad = cur.nonfinite();
         cur.template times<NCB>(smem, lane, acc);
-        O::store(reinterpret_cast<typename O::Raw*>(mine), acc, orr, r0, Wb, c0, ncols, lane, g, lr);
+        typename O::Raw* to = reinterpret_cast<typename O::Raw*>(mine);
+        O::store(to, acc, orr, r0, Wb, c0, ncols, lane, g, lr, [&] {
+            if constexpr (kB16) {
+                if (bad) whole_products<TIn, NJ, NCB>(to, bad, xr, r0, Wa, smem, lane, bias_of);
+            }
+        });
     }
 }
 
@@ -677,8 +743,16 @@ __global__ __launch_bounds__(kThreads, 2) void nc_query64_kernel(
             f32x4 acc[4];
 #pragma unroll
             for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const uint64_t bad = gm[h].nonfinite();
             gm[h].template times<4>(Em, lane, acc);
-            O::store(reinterpret_cast<typename O::Raw*>(mine), acc, dr, r0 + 16 * h, W, 0, W, lane, g, lr);
+            typename O::Raw* to = reinterpret_cast<typename O::Raw*>(mine);
+            O::store(to, acc, dr, r0 + 16 * h, W, 0, W, lane, g, lr, [&] {
+                if constexpr (kB16) {
+                    if (bad)
+                        whole_products<TIn, 4, 4>(to, bad, gr, r0 + 16 * h, W, Em, lane,
+                                                  [](int, int) { return f32x4{0.f, 0.f, 0.f, 0.f}; });
+                }
+            });
         }
     }
     o.combine(smem, records + (n * chunks + ci) * rec, W, W, 0, 0, false, w, g, lr);
@@ -795,8 +869,16 @@ __global__ __launch_bounds__(64 * NW) void nc_key64_kernel(
             f32x4 acc[4];
 #pragma unroll
             for (int cb = 0; cb < 4; ++cb) acc[cb] = bias[cb];
+            const uint64_t bad = vc.nonfinite();
             vc.template times<4>(Mk, lane, acc);
-            O::store(to, acc, dkr, r0, W, 0, W, lane, g, lr);
+            O::store(to, acc, dkr, r0, W, 0, W, lane, g, lr, [&] {
+                if constexpr (kB16) {
+                    if (bad)
+                        whole_products<TIn, 4, 4>(to, bad, vr, r0, W, Mk, lane, [&](int cb, int g) {
+                            return *reinterpret_cast<const f32x4*>(dAs + 16 * cb + 4 * g);
+                        });
+                }
+            });
         }
         X kc = kn;
         kc.turn(tx, lane, g, lr);
@@ -805,8 +887,15 @@ __global__ __launch_bounds__(64 * NW) void nc_key64_kernel(
             f32x4 acc[4];
 #pragma unroll
             for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const uint64_t bad = kc.nonfinite();
             kc.template times<4>(Mv, lane, acc);
-            O::store(to, acc, dvr, r0, W, 0, W, lane, g, lr);
+            O::store(to, acc, dvr, r0, W, 0, W, lane, g, lr, [&] {
+                if constexpr (kB16) {
+                    if (bad)
+                        whole_products<TIn, 4, 4>(to, bad, kr, r0, W, Mv, lane,
+                                                  [](int, int) { return f32x4{0.f, 0.f, 0.f, 0.f}; });
+                }
+            });
         }
     }
 }

@@ -100,3 +100,48 @@ def test_infinite_values_stay_where_they_are(race, cuda, dtype):
     keep[1, :, 7] = False
     assert torch.equal(got[keep], ref[keep])
     assert bool((got[1, :, 7] == float("inf")).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L, R, d", [(4, 16, 64), (2, 8, 40), (3, 16, 96), (5, 4, 36), (8, 32, 128)])
+def test_infinite_tokens_keep_their_sign(race, cuda, dtype, L, R, d):
+    # A token with one infinite value maps to that value's row of the matrix
+    # times an infinity: infinities of its signs, no NaN; tokens without one
+    # keep their bits.
+    say("nc inf tokens", dtype, L, R, d)
+    N, T, S = 2, 300, L * R
+    q, k, v, g = race.make_inputs(N, T, L, R, d, seed=11, dtype=dtype, grad_out=True)
+    q, k = q.reshape(N, T, S), k.reshape(N, T, S)
+    qc, kc, vc, gc = (x.to(cuda) for x in (q, k, v, g))
+    out, state = race.race_fused_fwd_with_state(qc, kc, vc, causal=False)
+    A, B = state[:, S * d:].double().cpu() + EPS, state[:, :S * d].reshape(N, S, d).double().cpu()
+    E = B / A[..., None]
+    dB = q.double().transpose(1, 2) @ g.double() / A[..., None]
+    hit = torch.arange(T) % 3 == 1  # every third token, the infinity in a column of its own
+
+    def spoil(x):
+        y, cols = x.clone(), torch.arange(T) % x.shape[-1]
+        y[:, hit, cols[hit]] = float("inf") * torch.where(torch.arange(T)[hit] % 2 == 0, 1.0, -1.0).to(y)
+        return y
+
+    def check_rows(got, clean, x, m, label):
+        # Expected: the sign of the infinity times the matrix row (x's column -> m's row).
+        cols = torch.arange(T) % x.shape[-1]
+        sign = torch.where(torch.arange(T) % 2 == 0, 1.0, -1.0)
+        want = (m[:, cols] * sign[:, None] * float("inf"))[:, hit]
+        assert torch.equal(got.double().cpu()[:, hit], want), label
+        assert torch.equal(got[:, ~hit], clean[:, ~hit]), label
+
+    # Q in the forward (the sums do not see it).
+    check_rows(race.race_fused_fwd(spoil(qc), kc, vc, causal=False), out, q, E, "out")
+    clean = race.race_noncausal_backward(qc, kc, vc, gc, state)
+    clean = [x.reshape(N, T, -1) for x in clean]
+    only = [True, False, False]
+    dq = race.race_noncausal_backward(qc, kc, vc, spoil(gc), state, need=only)[0]
+    check_rows(dq, clean[0], g, E.transpose(1, 2), "dQ alone")
+    dq = race.race_noncausal_backward(qc, kc, vc, spoil(gc), state)[0]
+    check_rows(dq, clean[0], g, E.transpose(1, 2), "dQ")
+    dk = race.race_noncausal_backward(qc, kc, spoil(vc), gc, state)[1]
+    check_rows(dk, clean[1], v, dB.transpose(1, 2), "dK")
+    dv = race.race_noncausal_backward(qc, spoil(kc), vc, gc, state)[2]
+    check_rows(dv, clean[2], k, dB, "dV")

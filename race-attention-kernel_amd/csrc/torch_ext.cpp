@@ -16,9 +16,9 @@
 //       -> (out, records or None, state or None, tile_tokens): the causal op
 //       with the hashing inside (race_hashed_fwd)
 //   module_forward(K, V, Q, planes_T, L, planes_per_table, causal, needs)
-//       -> (out, saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
+//       -> (out [M, B, H, T, d], saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
 //   module_backward(grad_out, saved, L, planes_per_table, causal, tile_tokens,
-//       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None
+//       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None; grad_out [M, B, H, T, d]
 //   hashed_supported(L, K, d) -> bool
 //   select_tile_tokens(N, T, L, R, d, bf16, causal, tile_tokens=0, kernel=0) -> int
 //   shape_supported(L, R, d) -> (supported, has_mfma)
@@ -576,9 +576,10 @@ int64_t select_tile_tokens(int64_t N, int64_t T, int64_t L, int64_t R, int64_t d
 
 // BatchedACE.forward (src/race_baseline.py:34-52) for K, V, Q [M, B, T, H, d]:
 // the heads' rows as streams, the hashing, and the op (causal: with the
-// hashing inside).  Returns the output [M, B, T, H, d] (a permuted view, as
-// the module's own), and with `needs` what module_backward reads: (K, Q, V
-// rows, planes, tile records) and the records' tile length, or (K, Q, V rows,
+// hashing inside).  Returns the output [M, B, H, T, d] (no view: what a custom
+// autograd function returns as one may not be changed in place; the module
+// permutes it), and with `needs` what module_backward reads: (K, Q, V rows,
+// planes, tile records) and the records' tile length, or (K, Q, V rows,
 // planes_T, probsK, probsQ, state).
 std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at::Tensor& K, const at::Tensor& V,
                                                                         const at::Tensor& Q,
@@ -603,16 +604,17 @@ std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at
         out = std::get<0>(r);
         if (needs) saved = {rows[0], rows[1], rows[2], pT, pk, pq, *std::get<1>(r)};
     }
-    return {out.view({M, B, H, T, d}).permute({0, 1, 3, 2, 4}), saved, tile};
+    return {at::_unsafe_view(out, {M, B, H, T, d}), saved, tile};
 }
 
 // Gradients of module_forward's rows [N, T, d] (None where not asked for) for
-// the upstream gradient [M, B, T, H, d] of the output.
+// the upstream gradient [M, B, H, T, d] of the output (dense once its heads are
+// permuted back, where the module's output had a dense gradient).
 std::tuple<c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>> module_backward(
     const at::Tensor& grad_out, const std::vector<at::Tensor>& saved, int64_t L, int64_t Kp, bool causal, int64_t tile,
     bool need_k, bool need_v, bool need_q) {
     const at::Tensor &K = saved[0], &Q = saved[1], &V = saved[2];
-    const at::Tensor g = streams_of({grad_out.to(V.scalar_type())})[0].view(V.sizes());
+    const at::Tensor g = streams_of({grad_out.to(V.scalar_type()).permute({0, 1, 3, 2, 4})})[0].view(V.sizes());
     c10::optional<at::Tensor> dq, dk, dv;
     at::Tensor pT;
     if (causal) {

@@ -250,7 +250,9 @@ def race_fused_fwd_hashed(K: torch.Tensor, Q: torch.Tensor, V: torch.Tensor, pla
 
 class ModuleRaceFunction(torch.autograd.Function):
     """BatchedACE.forward as one op: heads to streams, hashing and the op, and
-    their gradients, each direction one call into the binding.
+    their gradients, each direction one call into the binding.  The output is
+    [M, B, H, T, d]; the module permutes it outside, so that it may be changed
+    in place (the output of a custom function that is a view may not).
 
     What it saves is what the separate ops save: copies of the rows (so the
     inputs may change after the forward), the planes, and the forward's tile

@@ -100,3 +100,18 @@ def test_own_bucket_probs_are_used(race, cuda):
     ace = Uniform(64, 4, 4, 1, device=cuda, causal=False)
     mean = V.mean(2, keepdim=True).expand_as(V) * ace.L
     assert torch.allclose(ace(K, V, Q), mean, atol=1e-4)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("H", [1, 3])
+def test_output_may_be_changed_in_place(race, cuda, causal, H):
+    torch.manual_seed(2)
+    ace = race.BatchedACE(64, 4, 4, 1, device=cuda, causal=causal)
+    x = [torch.randn(1, 2, 40, H, 64, device=cuda).requires_grad_(True) for _ in range(3)]
+    out = ace(*x)
+    out += x[1]
+    out.mul_(2.0)
+    got = torch.autograd.grad(out.square().sum(), x)
+    ref = (ace(*x) + x[1]) * 2.0
+    assert torch.equal(out, ref)
+    assert all(torch.equal(a, b) for a, b in zip(got, torch.autograd.grad(ref.square().sum(), x)))

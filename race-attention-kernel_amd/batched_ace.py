@@ -8,8 +8,8 @@ corner softmax) and the hot span of lines 45-51 run in the same kernels, which
 hash the Q and K rows themselves (the reference's fused forward,
 src/race_fused_fwd.cu:80-146), so the bucket probabilities never reach memory.
 The non-causal module runs the hashing kernels and the non-causal op.  A
-causal module whose L, K, d_k the hashed kernels do not take, and a subclass
-with bucket_probs of its own, go through the separate ops.  Gradients reach
+causal module whose L, K, d_k the hashed kernels do not take, and a module
+whose bucket_probs is not the one below, go through the separate ops.  Gradients reach
 Khf, Qhf and Vhf on every path, as through the reference's torch composition;
 planes_T is a buffer there and here.
 """
@@ -44,7 +44,7 @@ class BatchedACE(nn.Module):
         M, B, T, H, dk = Khf.shape
         N = M * B * H
         hashed = self.causal and hashed_supported(self.L, self.K, dk)
-        own = getattr(self.bucket_probs, "__func__", None) is not BatchedACE.bucket_probs
+        own = getattr(self.bucket_probs, "__func__", None) is not _BUCKET_PROBS
         if not own and (hashed or not self.causal):
             out = ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal))
             return out.permute(0, 1, 3, 2, 4)
@@ -59,3 +59,8 @@ class BatchedACE(nn.Module):
             probsQ = self.bucket_probs(Qh2).contiguous()
             out2 = race_fused_fwd(probsQ, probsK, V2, self.causal)
         return out2.view(M, B, H, T, dk).permute(0, 1, 3, 2, 4)
+
+
+# The hashing the one-op forward stands for; any other bucket_probs (a
+# subclass's, an instance's, one put on the class) is called instead.
+_BUCKET_PROBS = BatchedACE.bucket_probs

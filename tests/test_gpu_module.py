@@ -115,3 +115,12 @@ def test_output_may_be_changed_in_place(race, cuda, causal, H):
     ref = (ace(*x) + x[1]) * 2.0
     assert torch.equal(out, ref)
     assert all(torch.equal(a, b) for a, b in zip(got, torch.autograd.grad(ref.square().sum(), x)))
+
+
+def test_bucket_probs_replaced_on_the_class_are_used(race, cuda, monkeypatch):
+    ace = race.BatchedACE(64, 4, 4, 1, device=cuda, causal=False)
+    monkeypatch.setattr(race.BatchedACE, "bucket_probs", lambda self, x2: torch.full(
+        (*x2.shape[:2], self.L, self.R), 1.0 / self.R, device=x2.device))
+    K, V, Q = (torch.randn(1, 1, 40, 2, 64, device=cuda) for _ in range(3))
+    mean = V.mean(2, keepdim=True).expand_as(V) * ace.L
+    assert torch.allclose(ace(K, V, Q), mean, atol=1e-4)

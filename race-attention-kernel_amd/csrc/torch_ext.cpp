@@ -15,7 +15,7 @@
 //   hashed_forward(K, Q, V, planes, L, tile_tokens=0, want_records=False, want_state=False)
 //       -> (out, records or None, state or None, tile_tokens): the causal op
 //       with the hashing inside (race_hashed_fwd)
-//   module_forward(K, V, Q, planes_T, L, planes_per_table, causal, needs)
+//   module_forward(K, V, Q, planes_T, L, planes_per_table, causal, need_k, need_v, need_q)
 //       -> (out [M, B, H, T, d], saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
 //   module_backward(grad_out, saved, L, planes_per_table, causal, tile_tokens,
 //       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None; grad_out [M, B, H, T, d]
@@ -578,13 +578,16 @@ int64_t select_tile_tokens(int64_t N, int64_t T, int64_t L, int64_t R, int64_t d
 // the heads' rows as streams, the hashing, and the op (causal: with the
 // hashing inside).  Returns the output [M, B, H, T, d] (no view: what a custom
 // autograd function returns as one may not be changed in place; the module
-// permutes it), and with `needs` what module_backward reads: (K, Q, V rows,
-// planes, tile records) and the records' tile length, or (K, Q, V rows,
-// planes_T, probsK, probsQ, state).
+// permutes it), and with a gradient to come what module_backward reads for it:
+// (V, K, Q rows, planes, tile records) and the records' tile length, or (V
+// rows, probsK, probsQ, state, then for K's and Q's gradients planes_T and the
+// rows of each that has one).
 std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at::Tensor& K, const at::Tensor& V,
                                                                         const at::Tensor& Q,
                                                                         const at::Tensor& planes_T, int64_t L,
-                                                                        int64_t Kp, bool causal, bool needs) {
+                                                                        int64_t Kp, bool causal, bool need_k,
+                                                                        bool need_v, bool need_q) {
+    const bool needs = need_k || need_v || need_q;
     const int64_t M = K.size(0), B = K.size(1), T = K.size(2), H = K.size(3), d = K.size(4), N = M * B * H;
     std::vector<at::Tensor> rows = streams_of({K, Q, V});
     for (at::Tensor& r : rows) r = r.view({N, T, d});
@@ -595,14 +598,17 @@ std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at
         const at::Tensor planes = planes_T.t().contiguous().to(at::kFloat);
         auto r = hashed_forward(rows[0], rows[1], rows[2], planes, L, 0, needs, false);
         out = std::get<0>(r);
-        if (needs) saved = {rows[0], rows[1], rows[2], planes, *std::get<1>(r)};
+        if (needs) saved = {rows[2], rows[0], rows[1], planes, *std::get<1>(r)};
         tile = std::get<3>(r);
     } else {
         const at::Tensor pT = planes_T.to(at::kFloat).contiguous();
         const at::Tensor pk = hash_probs(rows[0], pT, L, Kp), pq = hash_probs(rows[1], pT, L, Kp);
         auto r = forward(pq, pk, rows[2], false, 0, RACE_KERNEL_AUTO, needs);
         out = std::get<0>(r);
-        if (needs) saved = {rows[0], rows[1], rows[2], pT, pk, pq, *std::get<1>(r)};
+        if (needs) saved = {rows[2], pk, pq, *std::get<1>(r)};
+        if (need_k || need_q) saved.push_back(pT);
+        if (need_k) saved.push_back(rows[0]);
+        if (need_q) saved.push_back(rows[1]);
     }
     return {at::_unsafe_view(out, {M, B, H, T, d}), saved, tile};
 }
@@ -613,17 +619,21 @@ std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at
 std::tuple<c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>> module_backward(
     const at::Tensor& grad_out, const std::vector<at::Tensor>& saved, int64_t L, int64_t Kp, bool causal, int64_t tile,
     bool need_k, bool need_v, bool need_q) {
-    const at::Tensor &K = saved[0], &Q = saved[1], &V = saved[2];
+    const at::Tensor& V = saved[0];
     const at::Tensor g = streams_of({grad_out.to(V.scalar_type()).permute({0, 1, 3, 2, 4})})[0].view(V.sizes());
     c10::optional<at::Tensor> dq, dk, dv;
-    at::Tensor pT;
+    at::Tensor pT, K, Q;
     if (causal) {
+        K = saved[1];
+        Q = saved[2];
         pT = saved[3].t().contiguous();
         const at::Tensor pk = hash_probs(K, pT, L, Kp), pq = hash_probs(Q, pT, L, Kp);
         std::tie(dq, dk, dv) = causal_backward(pq, pk, V, g, need_q, need_k, need_v, tile, RACE_KERNEL_AUTO, saved[4]);
     } else {
-        pT = saved[3];
-        std::tie(dq, dk, dv) = noncausal_backward(saved[5], saved[4], V, g, saved[6], need_q, need_k, need_v, 0);
+        if (need_k || need_q) pT = saved[4];
+        if (need_k) K = saved[5];
+        if (need_q) Q = saved[need_k ? 6 : 5];
+        std::tie(dq, dk, dv) = noncausal_backward(saved[2], saved[1], V, g, saved[3], need_q, need_k, need_v, 0);
     }
     if (dk) dk = hash_probs_backward(K, pT, *dk, L, Kp);
     if (dq) dq = hash_probs_backward(Q, pT, *dq, L, Kp);
@@ -879,7 +889,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("tile_tokens") = 0, py::arg("want_records") = false, py::arg("want_state") = false);
     m.def("module_forward", &module_forward, "BatchedACE.forward -> (out, saved, tile_tokens)", py::arg("K"),
           py::arg("V"), py::arg("Q"), py::arg("planes_T"), py::arg("L"), py::arg("planes_per_table"),
-          py::arg("causal"), py::arg("needs"));
+          py::arg("causal"), py::arg("need_k"), py::arg("need_v"), py::arg("need_q"));
     m.def("module_backward", &module_backward, "Gradients of module_forward's rows -> (dK, dV, dQ)",
           py::arg("grad_out"), py::arg("saved"), py::arg("L"), py::arg("planes_per_table"), py::arg("causal"),
           py::arg("tile_tokens"), py::arg("need_k"), py::arg("need_v"), py::arg("need_q"));

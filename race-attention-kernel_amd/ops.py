@@ -254,15 +254,18 @@ class ModuleRaceFunction(torch.autograd.Function):
     [M, B, H, T, d]; the module permutes it outside, so that it may be changed
     in place (the output of a custom function that is a view may not).
 
-    What it saves is what the separate ops save: copies of the rows (so the
-    inputs may change after the forward), the planes, and the forward's tile
-    records (causal) or the probabilities and the state."""
+    What it saves is what the separate ops save: the rows, the planes, and the
+    forward's tile records (causal) or the probabilities and the state; the
+    non-causal backward reads K's and Q's rows, and the planes, only for
+    gradients of those, so they are saved only then.  The rows are
+    copies, so the inputs may change after the forward; with one head or one
+    token they are the inputs' own storage, and autograd raises if it changed."""
 
     @staticmethod
     def forward(ctx, Khf, Vhf, Qhf, planes_T, L, K, causal):
-        needs = any(ctx.needs_input_grad[:3])
-        out, saved, tile = _lib.ext().module_forward(Khf, Vhf, Qhf, planes_T, L, K, causal, needs)
-        if needs:
+        needs = ctx.needs_input_grad[:3]
+        out, saved, tile = _lib.ext().module_forward(Khf, Vhf, Qhf, planes_T, L, K, causal, *needs)
+        if any(needs):
             ctx.save_for_backward(*saved)
             ctx.args = (L, K, causal, tile)
             ctx.shapes = (Khf.shape, Vhf.shape, Qhf.shape)

@@ -124,3 +124,28 @@ def test_bucket_probs_replaced_on_the_class_are_used(race, cuda, monkeypatch):
     K, V, Q = (torch.randn(1, 1, 40, 2, 64, device=cuda) for _ in range(3))
     mean = V.mean(2, keepdim=True).expand_as(V) * ace.L
     assert torch.allclose(ace(K, V, Q), mean, atol=1e-4)
+
+
+def saved_floats(fn):
+    """Elements a call saves for its backward, each storage once."""
+    seen = {}
+
+    def pack(t):
+        seen[t.untyped_storage().data_ptr()] = t.untyped_storage().nbytes() // 4
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        out = fn()
+    return sum(seen.values()), out
+
+
+@pytest.mark.parametrize("need", [(True, False, False), (False, True, False), (False, False, True)])
+def test_rows_that_no_gradient_reads_are_not_saved(race, cuda, need):
+    # The separate ops keep the rows of a hashing only for its own gradient.
+    torch.manual_seed(3)
+    ace = race.BatchedACE(64, 4, 4, 1, device=cuda, causal=False)
+    x = [torch.randn(1, 2, 40, 3, 64, device=cuda).requires_grad_(n) for n in need]
+    got, _ = saved_floats(lambda: ace(*x))
+    ref, _ = saved_floats(lambda: composed(race, ace, *x))
+    assert got <= ref, (got, ref)
+    compare(race, ace, *x, need=need)

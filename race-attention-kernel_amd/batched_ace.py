@@ -46,7 +46,8 @@ class BatchedACE(nn.Module):
         hashed = self.causal and hashed_supported(self.L, self.K, dk)
         own = getattr(self.bucket_probs, "__func__", None) is not _BUCKET_PROBS
         if not own and (hashed or not self.causal):
-            out = ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal))
+            out = ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal),
+                                           torch.is_grad_enabled())
             return out.permute(0, 1, 3, 2, 4)
         Kh2 = Khf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
         Qh2 = Qhf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)

@@ -262,8 +262,10 @@ class ModuleRaceFunction(torch.autograd.Function):
     token they are the inputs' own storage, and autograd raises if it changed."""
 
     @staticmethod
-    def forward(ctx, Khf, Vhf, Qhf, planes_T, L, K, causal):
-        needs = ctx.needs_input_grad[:3]
+    def forward(ctx, Khf, Vhf, Qhf, planes_T, L, K, causal, grad_enabled):
+        # needs_input_grad tells which inputs require a gradient, also under
+        # no_grad (and in here gradients are always off).
+        needs = [grad_enabled and n for n in ctx.needs_input_grad[:3]]
         out, saved, tile = _lib.ext().module_forward(Khf, Vhf, Qhf, planes_T, L, K, causal, *needs)
         if any(needs):
             ctx.save_for_backward(*saved)
@@ -282,7 +284,7 @@ class ModuleRaceFunction(torch.autograd.Function):
             M, B, T, H, d = shape
             return None if g is None else g.view(M, B, H, T, d).permute(0, 1, 3, 2, 4)
 
-        return (*(heads(g, s) for g, s in zip(grads, ctx.shapes)), None, None, None, None)
+        return (*(heads(g, s) for g, s in zip(grads, ctx.shapes)), None, None, None, None, None)
 
 
 def hashed_supported(L: int, K: int, d: int) -> bool:

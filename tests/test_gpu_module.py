@@ -149,3 +149,32 @@ def test_rows_that_no_gradient_reads_are_not_saved(race, cuda, need):
     ref, _ = saved_floats(lambda: composed(race, ace, *x))
     assert got <= ref, (got, ref)
     compare(race, ace, *x, need=need)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_no_grad_keeps_nothing(race, ext, cuda, causal, monkeypatch):
+    # Inputs that require a gradient, in a forward without one: no state or
+    # records are asked for.
+    ace = race.BatchedACE(64, 4, 4, 1, device=cuda, causal=causal)
+    x = [torch.randn(1, 1, 40, 2, 64, device=cuda).requires_grad_(True) for _ in range(3)]
+    kept = []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(ext, name)
+            if name != "module_forward":
+                return f
+
+            def call(*a):
+                r = f(*a)
+                kept.append(len(r[1]))
+                return r
+
+            return call
+
+    monkeypatch.setattr(race.ops._lib, "ext", lambda: Spy())
+    with torch.no_grad():
+        out = ace(*x)
+    assert kept == [0] and not out.requires_grad
+    ace(*x)
+    assert kept[1] > 0

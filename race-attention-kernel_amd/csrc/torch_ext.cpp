@@ -7,7 +7,7 @@
 //   forward_carry(probsQ, probsK, V, state, tile_tokens=0, kernel=0, inplace=False)
 //       -> (out, state advanced over these tokens)
 //   noncausal_backward(probsQ, probsK, V, dOut, state, need_q, need_k, need_v,
-//                      tile_tokens=0) -> (dQ or None, dK or None, dV or None)
+//                      tile_tokens=0, kernel=0) -> (dQ or None, dK or None, dV or None)
 //   causal_backward(probsQ, probsK, V, dOut, need_q, need_k, need_v,
 //                   tile_tokens=0, kernel=0) -> (dQ or None, dK or None, dV or None)
 //   hash_probs(x, planes_T, L, K) -> [..., L, 2^K] bucket probabilities
@@ -264,7 +264,7 @@ std::tuple<at::Tensor, at::Tensor> forward_carry(const at::Tensor& q, const at::
 std::tuple<c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>>
 noncausal_backward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                    const at::Tensor& grad_out, const at::Tensor& state, bool need_q, bool need_k,
-                   bool need_v, int64_t tile_tokens) {
+                   bool need_v, int64_t tile_tokens, int64_t kernel = RACE_KERNEL_AUTO) {
     const race_shape sh = validate(q, k, v, "race_noncausal_backward");
     validate_like_v("race_noncausal_backward", "dOut", grad_out, v);
     const int64_t S = int64_t(sh.num_tables) * sh.num_buckets;
@@ -274,7 +274,7 @@ noncausal_backward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v
                      state.numel() == sh.num_streams * (S * sh.head_dim + S),
                  "state", "is not the forward's float32 [N, S*d + S] state on probsQ's device")
         .raise();
-    const race_options opts = make_options(tile_tokens, RACE_KERNEL_AUTO);
+    const race_options opts = make_options(tile_tokens, kernel);
     const c10::DeviceGuard guard(q.device());
     at::Tensor dq, dk, dv;
     if (need_q) dq = at::empty_like(q);
@@ -868,7 +868,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("noncausal_backward", &noncausal_backward, "Non-causal backward -> (dQ, dK, dV)",
           py::arg("probsQ"), py::arg("probsK"), py::arg("V"), py::arg("dOut"), py::arg("state"),
           py::arg("need_q") = true, py::arg("need_k") = true, py::arg("need_v") = true,
-          py::arg("tile_tokens") = 0);
+          py::arg("tile_tokens") = 0, py::arg("kernel") = 0);
     m.def("causal_backward", &causal_backward, "Causal backward -> (dQ, dK, dV)",
           py::arg("probsQ"), py::arg("probsK"), py::arg("V"), py::arg("dOut"),
           py::arg("need_q") = true, py::arg("need_k") = true, py::arg("need_v") = true,

@@ -57,6 +57,7 @@ class RaceFusedFunction(torch.autograd.Function):
         needs = any(ctx.needs_input_grad[:3])
         ctx.causal = bool(causal)
         ctx.tile_tokens = int(tile_tokens)
+        ctx.kernel = int(kernel)
         if needs and causal:
             # The scanned tile records (the prefix state at every tile start)
             # are kept, so the backward does not recompute them.
@@ -87,7 +88,7 @@ class RaceFusedFunction(torch.autograd.Function):
         q, k, v, state = ctx.saved_tensors
         grad_out = _dense(grad_out.to(v.dtype))
         dq, dk, dv = _lib.ext().noncausal_backward(q, k, v, grad_out, state, need_q, need_k,
-                                                  need_v, ctx.tile_tokens)
+                                                  need_v, ctx.tile_tokens, ctx.kernel)
         return dq, dk, dv, None, None, None
 
 
@@ -105,7 +106,8 @@ def race_fused_fwd(probsQ: torch.Tensor, probsK: torch.Tensor, V: torch.Tensor, 
         kernel: "auto", "valu" (fp32 vector kernels), "mfma" (matrix cores),
             "mfma_wg" (the workgroup matrix-core kernels) or "mfma_precise"
             (causal: the workgroup kernels with every product fp32-accurate
-            for bf16 inputs too; the backward keeps its own choice).
+            for bf16 inputs too).  The causal backward keeps its own choice;
+            the non-causal one runs "valu" where the forward did.
 
     Returns:
         out: [N, T, d] in V's dtype.
@@ -141,10 +143,11 @@ def race_fused_fwd_carry(probsQ, probsK, V, state, *, inplace: bool = False, til
 
 
 def race_noncausal_backward(probsQ, probsK, V, dOut, state, *, need=(True, True, True),
-                            tile_tokens: int = 0):
-    """(dQ, dK, dV) of the non-causal forward for upstream gradient dOut."""
+                            tile_tokens: int = 0, kernel: str | int = "auto"):
+    """(dQ, dK, dV) of the non-causal forward for upstream gradient dOut.  kernel:
+    "auto" (matrix cores for widths that are multiples of 4) or "valu"."""
     return _lib.ext().noncausal_backward(probsQ, probsK, V, _dense(dOut), state, *need,
-                                         tile_tokens)
+                                         tile_tokens, _kernel_id(kernel))
 
 
 def race_causal_backward(probsQ, probsK, V, dOut, *, need=(True, True, True),

@@ -88,6 +88,34 @@ def test_records_added_by_the_maps_or_before_them(race, cuda, dtype, tile):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L, R, d", [(4, 16, 64), (5, 20, 36), (4, 16, 128), (3, 5, 7)])
+@pytest.mark.parametrize("T, tile", [(200, 0), (500, 64), (700, 1024)])
+def test_vector_alu_backward(race, cuda, dtype, L, R, d, T, tile):
+    # kernel="valu" from the forward to its gradients: the folded passes (4
+    # tiles of 64 or one of 1024) and the finalize (8 of 64), each gradient
+    # alone, and for widths that have both families other bits than "auto".
+    say("nc-valu backward", dtype, L, R, d, T, tile)
+    N, S = 2, L * R
+    q, k, v, g = race.make_inputs(N, T, L, R, d, seed=T + d, dtype=dtype, grad_out=True)
+    leaves = [x.to(cuda).requires_grad_(True) for x in (q, k, v)]
+    out = race.race_fused_fwd(*leaves, causal=False, tile_tokens=tile, kernel="valu")
+    grads = torch.autograd.grad(out, leaves, g.to(cuda))
+    want, scale = exact(q, k, v, g)
+    check((out, *grads), want, scale, T, S, d, dtype, "valu")
+    qc, kc, vc, gc = (x.to(cuda) for x in (q, k, v, g))
+    _, state = race.race_fused_fwd_with_state(qc, kc, vc, causal=False, tile_tokens=tile, kernel="valu")
+    for need in ((True, True, True), (True, False, False), (False, True, False), (False, False, True), (False, True, True)):
+        part = race.race_noncausal_backward(qc, kc, vc, gc, state, need=need, tile_tokens=tile, kernel="valu")
+        for n, a, b in zip(need, part, grads):
+            assert torch.equal(a, b) if n else a is None
+    auto = race.race_noncausal_backward(qc, kc, vc, gc, state, tile_tokens=tile)
+    both = S % 4 == 0 and d % 4 == 0
+    assert all(torch.equal(a, b) for a, b in zip(auto, grads)) == (not both)
+    with pytest.raises(RuntimeError):
+        race.race_noncausal_backward(qc, kc, vc, gc, state, kernel="mfma")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_infinite_values_stay_where_they_are(race, cuda, dtype):
     # An infinity in one value column reaches that column's outputs only, as
     # infinities (the bf16 split of the staged matrix keeps them whole).

@@ -88,13 +88,13 @@ def test_shapes(race, oracle, cuda, dtype, L, R, d, T):
 
 @pytest.mark.parametrize("need", [(True, False, False), (False, True, False), (False, False, True),
                                   (True, True, False), (True, False, True), (False, True, True)])
-@pytest.mark.parametrize("T", [200, 500])
+@pytest.mark.parametrize("T", [200, 500, 1000])
 def test_only_requested_gradients(race, cuda, need, T):
     # At S = d = 64 the requests take different kernels (the query-side and
     # key-side passes, or the separate reduction, finalize and maps); every
-    # gradient must come out bit for bit the same either way.  T = 200 gives
-    # 4 tiles of 64 per stream (the key side sums the dE records itself),
-    # T = 500 gives 8 (after the finalize).
+    # gradient must come out bit for bit the same either way.  T = 200 and 500
+    # give 4 and 8 chunks per stream (the key side sums the dE records itself),
+    # T = 1000 gives 16 (after the finalize).
     say("needs-grad", need, T)
     q, k, v, g = (x.to(cuda) for x in race.make_inputs(2, T, 4, 16, 64, seed=3, grad_out=True))
     leaves = [x.clone().requires_grad_(n) for x, n in zip((q, k, v), need)]

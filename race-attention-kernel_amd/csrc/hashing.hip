@@ -290,8 +290,14 @@ size_t hash_lds_bytes(int dk, int L, int K) {
     return size_t(dk4 * lk_tier(L * K) + kHashRows * std::max(kXPitch, L * K + 1)) * sizeof(float);
 }
 
-hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, int64_t rows,
-                            int dk, int L, int K, int dtype, hipStream_t stream) {
+namespace {
+
+// Rows of one launch.  A launch of 2^32 threads or more wraps around without an
+// error; the kernels take up to two threads a row.
+constexpr int64_t kLaunchRows = int64_t(1) << 30;
+
+hipError_t hash_probs_rows(const void* x, const float* planes_T, void* probs, int64_t rows,
+                           int dk, int L, int K, int dtype, hipStream_t stream) {
     if (hash_rows_supported(x, probs, probs, dk, L, K, dtype))
         return launch_hash_rows(x, planes_T, nullptr, probs, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kHashRows - 1) / kHashRows));
@@ -324,8 +330,8 @@ hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, 
     return hipGetLastError();
 }
 
-hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const void* dprobs, void* dx,
-                                int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream) {
+hipError_t hash_probs_bwd_rows(const void* x, const float* planes_T, const void* dprobs, void* dx,
+                               int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream) {
     if (hash_rows_supported(x, dprobs, dx, dk, L, K, dtype))
         return launch_hash_rows(x, planes_T, dprobs, dx, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kThreads - 1) / kThreads));
@@ -346,6 +352,37 @@ hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const voi
     }
 #undef RACE_HASH_BWD
     return hipGetLastError();
+}
+
+// p advanced by `rows` rows of `width` values.
+const void* at_row(const void* p, int64_t rows, int width, int dtype) {
+    return static_cast<const char*>(p) + rows * width * (dtype == RACE_BF16 ? 2 : 4);
+}
+void* at_row(void* p, int64_t rows, int width, int dtype) {
+    return const_cast<void*>(at_row(static_cast<const void*>(p), rows, width, dtype));
+}
+
+}  // namespace
+
+hipError_t launch_hash_probs(const void* x, const float* planes_T, void* probs, int64_t rows,
+                            int dk, int L, int K, int dtype, hipStream_t stream) {
+    for (int64_t r = 0; r < rows; r += kLaunchRows) {
+        const hipError_t err = hash_probs_rows(at_row(x, r, dk, dtype), planes_T, at_row(probs, r, L << K, dtype),
+                                               std::min(rows - r, kLaunchRows), dk, L, K, dtype, stream);
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const void* dprobs, void* dx,
+                                int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream) {
+    for (int64_t r = 0; r < rows; r += kLaunchRows) {
+        const hipError_t err =
+            hash_probs_bwd_rows(at_row(x, r, dk, dtype), planes_T, at_row(dprobs, r, L << K, dtype),
+                                at_row(dx, r, dk, dtype), std::min(rows - r, kLaunchRows), dk, L, K, dtype, stream);
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
 }
 
 }  // namespace race

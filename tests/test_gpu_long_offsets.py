@@ -94,3 +94,36 @@ def test_bf16_offsets_past_2_to_the_31(race, oracle, cuda):
     say("bf16 2^32 elements last-stream tail max rel err", f"{err:.3e}")
     assert err <= 2e-2
     assert_bf16_floor(got, ref, vmax, "bf16 2^32 elements tail")
+
+
+def skip_unless_free(nbytes):
+    free, _ = torch.cuda.mem_get_info()
+    if free < nbytes * 1.02:
+        pytest.skip(f"needs {nbytes / 2**30:.0f} GiB of device memory, {free / 2**30:.0f} GiB free")
+
+
+def test_hashing_of_more_than_2_to_the_31_rows(race, cuda):
+    # More rows than one launch of the 16-row kernels holds threads for.
+    dk, L, K = 4, 2, 2
+    rows = 2 ** 31 + 200
+    skip_unless_free(rows * 2 * 2 * (dk + L * (1 << K)))
+    say("hash rows", rows)
+    gen = torch.Generator(device=cuda).manual_seed(31)
+    planes_T = torch.randn(dk, L * K, generator=gen, device=cuda)
+    x = torch.zeros(rows, dk, dtype=torch.bfloat16, device=cuda)
+    spans = [slice(0, 300), slice(2 ** 30 - 300, 2 ** 30 + 300), slice(rows - 600, rows)]
+    for s in spans:
+        x[s] = torch.randn(x[s].shape, generator=gen, device=cuda).to(x.dtype)
+    probs = race.race_hash_probs(x, planes_T, L, K)
+    for s in spans:
+        assert torch.equal(probs[s], race.race_hash_probs(x[s].clone(), planes_T, L, K)), s
+    g = torch.zeros_like(probs)
+    for s in spans:
+        g[s] = torch.randn(g[s].shape, generator=gen, device=cuda).to(g.dtype)
+    del probs
+    ext = race.ops._lib.ext()
+    dx = ext.hash_probs_backward(x, planes_T, g, L, K)
+    for s in spans:
+        assert torch.equal(dx[s], ext.hash_probs_backward(x[s].clone(), planes_T, g[s].clone(), L, K)), s
+    del x, g, dx
+    torch.cuda.empty_cache()

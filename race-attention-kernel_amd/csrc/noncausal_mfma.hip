@@ -40,6 +40,8 @@
 //     -> 10 / 9 / 14 / 14: launches of one workgroup per stream, bound by the
 //     latency of staging, the loop's few steps and the launch itself.
 // Other widths (S 12 .. 256, d 20 .. 128) ran 1.2x (100 x 36, fp32) to 9x.
+#include <algorithm>
+
 #include "mfma_common.h"
 
 namespace race {
@@ -903,9 +905,12 @@ __global__ __launch_bounds__(64 * NW) void nc_key64_kernel(
 // Values per lane for a width: 16 lanes cover it, or a block of 64.
 int lane_values(int W) { return W <= 16 ? 1 : W <= 32 ? 2 : 4; }
 
-// Tokens per workgroup of a map, whole 16-token tiles.
+// Tokens per workgroup of a map, whole 16-token tiles.  The blocks of all
+// streams are one grid dimension, and a launch of 2^32 threads or more wraps
+// around without an error.
 int map_wg_tokens(const Problem& p, int slices) {
-    const int64_t per = nc_blocks_per_stream(p.N * slices, p.T, p.dtype, kMapMaxTokens);
+    const int64_t most = ((int64_t(1) << 32) - 1) / (64 * kMapWaves) / p.N;
+    const int64_t per = std::min(most, nc_blocks_per_stream(p.N * slices, p.T, p.dtype, kMapMaxTokens));
     return int(((p.T + per - 1) / per + 15) / 16 * 16);
 }
 

@@ -127,3 +127,19 @@ def test_hashing_of_more_than_2_to_the_31_rows(race, cuda):
         assert torch.equal(dx[s], ext.hash_probs_backward(x[s].clone(), planes_T, g[s].clone(), L, K)), s
     del x, g, dx
     torch.cuda.empty_cache()
+
+
+def test_noncausal_maps_of_more_than_2_to_the_33_tokens(race, cuda):
+    # More token blocks over all streams than one launch holds threads for.
+    # Constant inputs (probsQ is probsK): every output is the value, 2.
+    N, T, L, R, d = 65535, 131200, 1, 4, 4
+    skip_unless_free(3 * N * T * 2 * d)
+    say("nc map", N, T)
+    p = torch.full((N, T, L, R), 0.25, dtype=torch.bfloat16, device=cuda)
+    v = torch.full((N, T, d), 2.0, dtype=torch.bfloat16, device=cuda)
+    out = race.race_fused_fwd(p, p, v, causal=False)
+    del p, v
+    for n in range(0, N, 4096):  # in pieces: no temporaries of the whole
+        assert bool((out[n:n + 4096] == 2.0).all()), n
+    del out
+    torch.cuda.empty_cache()

@@ -12,6 +12,8 @@
 // for the kernels that follow: three tensors of 131072 fp32 rows of 64 (201 MB
 // moved) 47 -> 33 us with the nontemporal reads, 37 with nontemporal writes
 // too; torch's permuted copies took 50.
+#include <algorithm>
+
 #include "race_internal.h"
 
 namespace race {
@@ -19,6 +21,9 @@ namespace {
 
 constexpr int kPackChunks = 1024;  // 16-byte chunks per workgroup: 4 per thread
 constexpr int kPackUnroll = kPackChunks / kThreads;
+// Workgroups of a batch in one launch: one of 2^32 threads or more wraps around
+// without an error.
+constexpr int64_t kPackLaunch = int64_t(1) << 23;
 
 typedef uint32_t Chunk __attribute__((ext_vector_type(4)));
 
@@ -28,14 +33,16 @@ struct PackArgs {
 };
 
 // vec: 16-byte chunks per row (1 << shift where that is a power of two, else
-// shift < 0); tokens: rows per workgroup, at most kPackChunks chunks.
+// shift < 0); tokens: rows per workgroup, at most kPackChunks chunks; first: the
+// launch's first workgroup of a batch.
 __global__ __launch_bounds__(kThreads) void pack_heads_kernel(PackArgs a, int64_t T, int H, int vec, int shift,
-                                                              int tokens) {
+                                                              int tokens, unsigned first) {
     const Chunk* src = a.src[blockIdx.z];
     Chunk* dst = a.dst[blockIdx.z];
     const int64_t b = blockIdx.y;
-    const int h = int(blockIdx.x % unsigned(H));
-    const int64_t t0 = int64_t(blockIdx.x / unsigned(H)) * tokens;
+    const unsigned wg = first + blockIdx.x;
+    const int h = int(wg % unsigned(H));
+    const int64_t t0 = int64_t(wg / unsigned(H)) * tokens;
     const int chunks = int(min<int64_t>(tokens, T - t0)) * vec;
     const int64_t from = ((b * T + t0) * H + h) * vec, to = ((b * H + h) * T + t0) * vec;
     Chunk v[kPackUnroll];
@@ -64,9 +71,14 @@ hipError_t launch_pack_heads(const void* const* src, void* const* dst, int count
     const int vec = row_bytes / 16;
     const int shift = (vec & (vec - 1)) == 0 ? __builtin_ctz(vec) : -1;
     const int tokens = kPackChunks / vec;
-    const dim3 grid(unsigned((T + tokens - 1) / tokens * H), unsigned(batch), unsigned(count));
-    pack_heads_kernel<<<grid, kThreads, 0, stream>>>(a, T, H, vec, shift, tokens);
-    return hipGetLastError();
+    const int64_t wgs = (T + tokens - 1) / tokens * H;
+    for (int64_t w = 0; w < wgs; w += kPackLaunch) {
+        const dim3 grid(unsigned(std::min(wgs - w, kPackLaunch)), unsigned(batch), unsigned(count));
+        pack_heads_kernel<<<grid, kThreads, 0, stream>>>(a, T, H, vec, shift, tokens, unsigned(w));
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
 }
 
 }  // namespace race

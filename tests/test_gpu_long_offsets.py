@@ -12,6 +12,8 @@ with the distribution of the BASELINE configurations.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -143,3 +145,19 @@ def test_noncausal_maps_of_more_than_2_to_the_33_tokens(race, cuda):
         assert bool((out[n:n + 4096] == 2.0).all()), n
     del out
     torch.cuda.empty_cache()
+
+
+def test_packing_more_than_2_to_the_24_heads(race, cuda):
+    # The C entry's copy with a run of one head per workgroup, more of them
+    # than one launch holds threads for.
+    T, H, d = 2, 2 ** 24 + 5, 4
+    say("pack heads", T, H)
+    src = torch.randn(T, H, d, device=cuda)
+    dst = torch.zeros(H, T, d, device=cuda)
+    from race_attention_kernel_amd import abi
+
+    args = [(ctypes.c_void_p * 1)(x.data_ptr()) for x in (src, dst)]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    status = abi.lib().race_pack_heads(args[0], args[1], 1, ctypes.c_int64(1), ctypes.c_int64(T), H, d, 0, stream)
+    assert status == 0
+    assert torch.equal(dst, src.transpose(0, 1))

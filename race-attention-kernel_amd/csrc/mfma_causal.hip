@@ -480,11 +480,9 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     const dim3 grid(unsigned(p.tiles), unsigned(p.N));
     hipError_t err = hipSuccess;
     if constexpr (S == 64 && D == 64) {
-        // One launch; the marks of the three keep their places.  (A state must not
-        // be written over the carried one while other workgroups still read it.)
+        // One launch.  (A state must not be written over the carried one while
+        // other workgroups still read it.)
         if (short_prefixes(p) && (!state || state != p.init)) {
-            if (marks && ((err = marks->mark(stream)) != hipSuccess || (err = marks->mark(stream)) != hipSuccess))
-                return err;
             constexpr size_t kQuad = kQuadLdsFloats * sizeof(float);
             constexpr size_t kLds = size_t(GO::kOutputLds) > kQuad ? size_t(GO::kOutputLds) : kQuad;
             const dim3 fused(unsigned(p.tiles + (state ? 1 : 0)), unsigned(p.N));

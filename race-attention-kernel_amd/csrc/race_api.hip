@@ -1012,8 +1012,10 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
         else
             RACE_TRY(launch_tile_outer_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         RACE_TRY(marks->mark(stream));
-        if (!short_prefixes(p)) RACE_TRY(launch_tile_scan(fwd_ws, nullptr, p, stream));
-        RACE_TRY(marks->mark(stream));
+        if (!short_prefixes(p)) {
+            RACE_TRY(launch_tile_scan(fwd_ws, nullptr, p, stream));
+            RACE_TRY(marks->mark(stream));
+        }
         fwd_rec = fwd_ws;
     }
     if (use_mfma && !pl.blocked()) {

@@ -8,6 +8,8 @@ the backward from the saved records against the one that recomputes them.
 """
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -66,3 +68,30 @@ def test_saved_records_and_recomputed_ones_give_the_same_bits(race, ext, cuda, d
     saved = ext.causal_backward(q, k, v, g, True, True, True, used, 0, records)
     again = ext.causal_backward(q, k, v, g, True, True, True, used, 0, None)
     assert all(torch.equal(a, b) for a, b in zip(saved, again))
+
+
+@pytest.mark.parametrize("T, tile, fwd, bwd", [(512, 64, 1, 4), (576, 64, 1, 4), (577, 64, 3, 5)])
+def test_every_launch_is_marked_once(race, cuda, T, tile, fwd, bwd):
+    # An event before the first launch and after every one, none for launches
+    # that a short sequence does without.
+    from race_attention_kernel_amd import abi
+
+    q, k, v, g = race.make_inputs(2, T, 4, 16, 64, seed=T, device=cuda, grad_out=True)
+    out, dq, dk, dv = (torch.empty_like(x) for x in (v, q, k, v))
+    sh, opts = abi.shape(2, T, 4, 16, 64), abi.options(tile, 0)
+    events = [torch.cuda.Event(enable_timing=True) for _ in range(16)]
+    stream = torch.cuda.current_stream()
+    for e in events:
+        e.record(stream)  # creates the handle
+    handles = (ctypes.c_void_p * 16)(*(e.cuda_event for e in events))
+    status, nbytes, _, _ = abi.fwd_workspace_bytes(sh, True, opts)
+    ws = torch.empty(nbytes // 4, device=cuda)
+    status, n = abi.fwd_profiled(*(x.data_ptr() for x in (q, k, v, out)), None, sh, True, opts, ws.data_ptr(),
+                                 nbytes, stream.cuda_stream, handles)
+    assert (status, n) == (0, fwd + 1)
+    status, nbytes = abi.causal_bwd_workspace_bytes(sh, opts)
+    ws = torch.empty(nbytes // 4, device=cuda)
+    status, n = abi.causal_bwd_profiled(*(x.data_ptr() for x in (q, k, v, g, dq, dk, dv)), sh, opts, ws.data_ptr(),
+                                        nbytes, stream.cuda_stream, handles)
+    assert (status, n) == (0, bwd + 1)
+    torch.cuda.synchronize()

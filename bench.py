@@ -92,13 +92,11 @@ WORKLOADS = {
 PHASES = {
     (True, "valu"): ["tile_sums", "tile_scan", "output_pass_valu"],
     (False, "valu"): ["tile_sums", "tile_reduce", "token_map"],
+    (False, "mfma"): ["tile_sums", "tile_reduce", "token_map"],
     (True, "mfma"): ["tile_sums_mfma", "tile_scan", "output_pass_mfma"],
     (True, "hashed"): ["hashed_sums", "tile_scan", "hashed_output"],
     (True, "single"): ["single_arm", "single_pass"],
 }
-# Non-causal forwards with at most this many tiles per stream add the tile
-# records inside the map (no tile_reduce launch), as race_api.hip does.
-NONCAUSAL_FOLD_TILES = 4
 # Backward launch sequences (every gradient requested).
 BWD_PHASES = {
     True: ["bwd_tile_sums", "tile_scan", "bwd_dq", "suffix_scan", "bwd_dkv"],
@@ -106,7 +104,20 @@ BWD_PHASES = {
 }
 
 
-def causal_bwd_phases(S: int, d: int, es: int, whole_streams: bool = False) -> list:
+def fwd_phases(causal: bool, family: str, launches: int) -> list:
+    """The forward's launches by name, from the number the library marked: all
+    of PHASES, a non-causal forward whose maps add the tile records themselves
+    (no tile_reduce), or a short causal one whose output workgroups form their
+    own prefixes (one launch)."""
+    names = PHASES.get((causal, family), [])
+    if not causal and launches == 2:
+        return [n for n in names if n != "tile_reduce"]
+    if (causal, family, launches) == (True, "mfma", 1):
+        return ["output_pass_short"]
+    return names
+
+
+def causal_bwd_phases(S: int, d: int, es: int, whole_streams: bool = False, launches: int = 0) -> list:
     """The causal backward's launches as race_api.hip issues them (starting
     from the inputs): one 64 x 64 block at S = d = 64; with bf16 tokens, d =
     128 and S = 128 or 256, the forward walks of every 128-bucket block
@@ -114,9 +125,11 @@ def causal_bwd_phases(S: int, d: int, es: int, whole_streams: bool = False) -> l
     records, then a backward walk per block; other shapes get generic
     names.  With `whole_streams` (the streams times the blocks fill the
     device's CUs, or one tile per stream) the forward walks go through whole
-    streams and the forward's tile sums and scan are not run."""
+    streams and the forward's tile sums and scan are not run.  `launches`, when
+    given, is the number the library marked: a short sequence's prefixes at S =
+    d = 64 take one launch and no scan."""
     if S == 64 and d == 64:
-        return BWD_PHASES[True]
+        return ["bwd_prefixes"] + BWD_PHASES[True][2:] if launches == 4 else BWD_PHASES[True]
     if es == 2 and d == 128 and S in (128, 256):
         names = [] if whole_streams else ["bwd_tile_sums", "tile_scan"]
         names += ["bwd_dq_walks", "suffix_scan_blocks"]
@@ -124,14 +137,12 @@ def causal_bwd_phases(S: int, d: int, es: int, whole_streams: bool = False) -> l
     return []
 
 
-def noncausal_bwd_phases(S: int, d: int, tiles: int) -> list:
-    """The non-causal backward's launches as race_api.hip issues them: at
-    S = d = 64 the query side and the key side, with the finalize between
-    them past NONCAUSAL_FOLD_TILES tiles per stream; the five passes
-    otherwise."""
+def noncausal_bwd_phases(S: int, d: int, launches: int) -> list:
+    """The non-causal backward's launches by name, from the number the library
+    marked: at S = d = 64 the query side and the key side, with the finalize
+    between them when there are three; the five passes otherwise."""
     if S == 64 and d == 64:
-        mid = ["bwd_finalize"] if tiles > NONCAUSAL_FOLD_TILES else []
-        return ["query_grad"] + mid + ["key_grad"]
+        return ["query_grad"] + (["bwd_finalize"] if launches == 3 else []) + ["key_grad"]
     return BWD_PHASES[False]
 
 
@@ -283,11 +294,13 @@ def phase_bytes(name: str, cfg, T: int, es: int, tiles: int, rec: int) -> float:
         "tile_reduce": state,
         "output_pass_valu": es * (2 * S + 2 * d) * NT,
         "output_pass_mfma": es * (2 * S + 2 * d) * NT,
+        "output_pass_short": es * (2 * S + 2 * d) * NT,
         "single_arm": 4.0 * cfg.N * tiles,         # zeroes one flag per tile
         "single_pass": es * (2 * S + 2 * d) * NT,  # q, k, v read once -> out
         "token_map": es * (S + d) * NT,
         # backward: each launch's own operands (reads) and outputs (writes)
         "bwd_tile_sums": es * (S + d) * NT,
+        "bwd_prefixes": es * (S + d) * NT,
         "bwd_dq": es * (3 * S + 2 * d) * NT,       # q, k, v, dOut -> dQ
         "suffix_scan": 2 * state,
         "bwd_dkv": es * (3 * S + 3 * d) * NT,      # q, k, v, dOut -> dK, dV
@@ -727,6 +740,8 @@ def measure(args, T: int) -> dict:
     if cfg.causal and (kernel_id in (2, 3, 6) or (kernel_id == 0 and race.ops._lib.ext().shape_supported(
             cfg.L, cfg.R, cfg.d)[1])):
         family = "mfma"
+    if not cfg.causal and kernel_id == 0 and cfg.S % 4 == 0 and cfg.d % 4 == 0:
+        family = "mfma"
     if cfg.causal and kernel_id == race.ops.KERNELS["single"]:
         family = "single"
     ws = torch.empty(max(ws_bytes // 4, 1), device=dev, dtype=torch.float32)
@@ -825,6 +840,8 @@ def measure(args, T: int) -> dict:
                 check(abi.noncausal_bwd(*bptrs, sptr, *gptrs, sh, bopts, bws.data_ptr(), bws_bytes,
                                         stream))
 
+    marked = {"fwd": 0, "bwd": 0}  # launches the last profiled step's calls marked
+
     def profiled(evs):
         n_used = 0
         if run_hashed:
@@ -844,6 +861,7 @@ def measure(args, T: int) -> dict:
             st_, n = abi.fwd_profiled(*fwd_ptrs(), sptr, sh, cfg.causal, opts, ws.data_ptr(), ws_bytes,
                                       stream, tail)
             check(st_)
+            marked["fwd"] = n - 1
             n_used += n
         if run_bwd:
             tail = (ctypes.c_void_p * (len(evs) - n_used)).from_buffer(evs, n_used * ctypes.sizeof(ctypes.c_void_p))
@@ -854,23 +872,9 @@ def measure(args, T: int) -> dict:
                 st_, n = abi.noncausal_bwd_profiled(*bptrs, sptr, *gptrs, sh, bopts, bws.data_ptr(),
                                                     bws_bytes, stream, tail)
             check(st_)
+            marked["bwd"] = n - 1
             n_used += n
         return n_used
-
-    fwd_names = PHASES.get((cfg.causal, family), [])
-    if not cfg.causal and tiles <= NONCAUSAL_FOLD_TILES:
-        fwd_names = [n for n in fwd_names if n != "tile_reduce"]
-    names = []
-    if run_hashed:
-        names += PHASES[(True, "hashed")]
-    if run_hash:
-        names += ["hash_q", "hash_k"]
-    if run_fwd:
-        names += fwd_names
-    if run_bwd:
-        whole = tiles == 1 or cfg.N * (cfg.S // 128) >= torch.cuda.get_device_properties(dev).multi_processor_count
-        names += (causal_bwd_phases(cfg.S, cfg.d, es, whole) if cfg.causal
-                  else noncausal_bwd_phases(cfg.S, cfg.d, tiles))
 
     if args.calibrate_copy:
         # A plain copy of known size: its FETCH_SIZE / WRITE_SIZE counters give
@@ -963,7 +967,18 @@ def measure(args, T: int) -> dict:
     n_gaps = n_events - 1
     gaps = [statistics.fmean(events.elapsed_ms(ev[j], ev[j + 1]) for ev in per_step)
             for j in range(n_gaps)]
-    n_fwd = len(fwd_names) if run_fwd else 0
+    n_fwd = marked["fwd"]
+    names = []
+    if run_hashed:
+        names += PHASES[(True, "hashed")]
+    if run_hash:
+        names += ["hash_q", "hash_k"]
+    if run_fwd:
+        names += fwd_phases(cfg.causal, family, n_fwd)
+    if run_bwd:
+        whole = tiles == 1 or cfg.N * (cfg.S // 128) >= torch.cuda.get_device_properties(dev).multi_processor_count
+        names += (causal_bwd_phases(cfg.S, cfg.d, es, whole, marked["bwd"]) if cfg.causal
+                  else noncausal_bwd_phases(cfg.S, cfg.d, marked["bwd"]))
     if run_fwd and run_bwd:
         gaps = gaps[:n_fwd] + gaps[n_fwd + 1:]
     if run_hash:  # the forward's first event follows the hashing's last one

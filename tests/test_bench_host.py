@@ -45,13 +45,26 @@ def test_sweep_lengths_cover_cfg1_and_cfg2():
     assert b.GPU_SWEEP_T == [512 << i for i in range(8)]
 
 
+def test_forward_launch_names_follow_the_library():
+    # The library marks every launch: a non-causal forward reduces the tile
+    # records in a launch of its own or in its maps, a short causal one forms
+    # its prefixes in the output workgroups.
+    b = load_bench()
+    for family in ("valu", "mfma"):
+        assert b.fwd_phases(False, family, 3) == ["tile_sums", "tile_reduce", "token_map"]
+        assert b.fwd_phases(False, family, 2) == ["tile_sums", "token_map"]
+    assert b.fwd_phases(True, "mfma", 3) == ["tile_sums_mfma", "tile_scan", "output_pass_mfma"]
+    assert b.fwd_phases(True, "mfma", 1) == ["output_pass_short"]
+
+
 def test_noncausal_backward_launch_names_follow_the_library():
-    # race_api.hip: at S = d = 64 the query side and the key side (with the
-    # finalize between them past 4 tiles per stream); five passes otherwise.
+    # race_api.hip: at S = d = 64 the query side and the key side, with the
+    # finalize between them when the key side does not add the records itself;
+    # five passes otherwise.
     b = load_bench()
     assert b.noncausal_bwd_phases(64, 64, 2) == ["query_grad", "key_grad"]
-    assert b.noncausal_bwd_phases(64, 64, 8) == ["query_grad", "bwd_finalize", "key_grad"]
-    assert b.noncausal_bwd_phases(256, 128, 2) == b.BWD_PHASES[False]
+    assert b.noncausal_bwd_phases(64, 64, 3) == ["query_grad", "bwd_finalize", "key_grad"]
+    assert b.noncausal_bwd_phases(256, 128, 5) == b.BWD_PHASES[False]
 
 
 def test_causal_backward_launch_names_follow_the_library():
@@ -61,6 +74,7 @@ def test_causal_backward_launch_names_follow_the_library():
     # backward walk per block; other shapes get generic names.
     b = load_bench()
     assert b.causal_bwd_phases(64, 64, 4) == b.BWD_PHASES[True]
+    assert b.causal_bwd_phases(64, 64, 4, launches=4) == ["bwd_prefixes", "bwd_dq", "suffix_scan", "bwd_dkv"]
     assert b.causal_bwd_phases(256, 128, 2) == [
         "bwd_tile_sums", "tile_scan", "bwd_dq_walks", "suffix_scan_blocks", "bwd_dkv_pair0",
         "bwd_dkv_pair1"]

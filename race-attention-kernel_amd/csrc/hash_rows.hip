@@ -37,13 +37,14 @@ namespace race {
 namespace {
 
 using mfma::f32x4;
+using mfma::kOutside;
+using mfma::mfma4;
 using mfma::u32x2;
 using mfma::u32x4;
 
 constexpr int kGroups = 2;                          // 16-row groups per wave
 constexpr int kWaves = kThreads / 64;
 constexpr int kWgRows = 16 * kGroups * kWaves;      // rows per workgroup
-constexpr int kOutside = 0x7ffffff0;                // past any buffer view
 
 // Which table and plane the slot `row` (0..15) of slot block `b` carries.
 template <int K>
@@ -166,7 +167,7 @@ __device__ __forceinline__ f32x4 project(const f32x4* __restrict__ pa, const Row
     for (int j = 0; j < NJ; ++j) {
         const f32x4 p = pa[(b * NJ + j) * 64 + lane], xv = x[j].f32();
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[e], xv[e], a[e], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) a[e] = mfma4(p[e], xv[e], a[e]);
     }
     return (a[0] + a[1]) + (a[2] + a[3]);
 }
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(kThreads) void hash_rows_bwd_kernel(
                     const f32x4 p = pt[((b + h) * NJ + j) * 64 + lane];
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[e], dp[4 * h + e], acc[j], 0, 0, 0);
+                        acc[j] = mfma4(p[e], dp[4 * h + e], acc[j]);
                 }
         }
 #pragma unroll

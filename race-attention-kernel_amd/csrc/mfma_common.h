@@ -34,6 +34,11 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// fp32: one value of the contraction per lane group.
+__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 // acc += A B with optional hi/lo operands: lo*hi and hi*lo first, then hi*hi.
 template <bool kSplit>
 __device__ __forceinline__ f32x4 mfma3(const bf16x8& ah, const bf16x8& al, const bf16x8& bh,
@@ -98,6 +103,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, in
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, int(bytes),
                                              0x00020000);
 }
+// A byte offset past the end of every such view.
+constexpr int kOutside = 0x7ffffff0;
 // Cache policy bits of buffer loads and stores (the instruction's aux field):
 // 0 = default, 2 = nontemporal (`nt`).  Streaming reads with `nt` run at about
 // 7.1 TB/s on MI355X against 6.3 TB/s without it; each kernel picks its own.

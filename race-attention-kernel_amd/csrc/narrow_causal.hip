@@ -41,14 +41,11 @@ namespace race {
 namespace {
 
 using mfma::f32x4;
+using mfma::kOutside;
+using mfma::mfma4;
 using mfma::u32x4;
 
 constexpr int kWaves = kThreads / 64;
-constexpr int kOutside = 0x7ffffff0;  // past any buffer view
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 // E consecutive values at byte offset `off`, as floats.
 template <typename TIn, int E>

@@ -49,23 +49,20 @@ namespace {
 
 using mfma::bf16x8;
 using mfma::f32x4;
+using mfma::kOutside;
 using mfma::mfma16;
+using mfma::mfma4;
 using mfma::u32x2;
 using mfma::u32x4;
 
 constexpr int kWaves = kThreads / 64;  // waves of a reduction workgroup
 constexpr int kMapWaves = 8;            // waves of a map workgroup: they share one staged matrix
 constexpr int64_t kMapMaxTokens = 1024;
-constexpr int kOutside = 0x7ffffff0;  // past any buffer view
 // Tokens a wave takes at a time: one fp32 MFMA tile, or the 32-token
 // contraction of a bf16 one.
 template <typename TIn>
 constexpr int kStep = sizeof(TIn) == 4 ? 16 : 32;
 constexpr int kNcStorePolicy = 2;  // nontemporal: the results are not read again here
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 // E consecutive elements of a token row.
 template <typename TIn, int E>

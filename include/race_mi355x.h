@@ -235,8 +235,9 @@ race_status race_fwd_carry_workspace_bytes(const race_shape* shape, const race_o
  * receives init_state plus the sums over all T tokens and may equal
  * init_state (an in-place step).  Splitting a sequence anywhere and carrying
  * the state gives the unsplit result up to fp32 rounding.  Short calls
- * (decode: T <= RACE_DECODE_TOKENS) run one launch with one workgroup per
- * stream and no workspace; longer ones run race_fwd's causal kernels with the
+ * (decode: T <= RACE_DECODE_TOKENS) run one launch and no workspace, with one
+ * workgroup per stream (two for d > 64 and up to 128 streams, unless state is
+ * init_state); longer ones run race_fwd's causal kernels with the
  * tile scan started from init_state.  The reference has no kernel for this. */
 race_status race_fwd_carry(const void* probsQ, const void* probsK, const void* V, void* out,
                            const float* init_state, float* state, const race_shape* shape,

@@ -419,8 +419,8 @@ hipError_t launch_tile_sums_direct(const void* k, const void* v, float* records,
             cache_kept_rows(p), nullptr);
         return hipGetLastError();
     }
-    // bf16 S = d = 64: a workgroup per tile from 256 tokens on, whose sixteen-token
-    // strips keep each wave busy; below, one wave per tile (N = 256, T = 1000: tile
+    // bf16 S = d = 64: a workgroup per tile from 256 tokens on, two 32-token steps
+    // or more for each wave; below, one wave per tile (N = 256, T = 1000: tile
     // 128 sums 19.7 us by workgroups, 15.3 by waves; tile 256 equal).
     if (p.dtype == RACE_BF16 && p.S == 64 && p.d == 64 && p.tile >= 256)
         return launch_tile_sums_b16(k, v, records, p, stream);

@@ -11,8 +11,9 @@
 // bf16 tokens: v_mfma_f32_16x16x32_bf16, sixteen times that rate.  A reduction's
 // products of two bf16 values are exact in its fp32 sums; a map's fp32 matrix
 // is split into three bf16 terms that add up to it exactly (8 bits each,
-// truncated), so its products are the fp32 ones too (for finite tokens; those
-// with an infinity or NaN take fp32 products, whole_products).
+// truncated; below 2^-110 to within 2^-133, the least a bf16 term holds), so
+// its products are the fp32 ones too (for finite tokens; those with an infinity
+// or NaN take fp32 products, whole_products).
 // The token rows never go through workgroup-wide LDS staging: a wave loads
 // whole rows into registers and, where the products want the other layout,
 // turns 16 or 32 rows through a piece of LDS of its own, without barriers.
@@ -377,7 +378,7 @@ template <int NJ, int NCB, bool kB16>
 constexpr int kMatrixFloats = kB16 ? 32 * ((NJ + 1) / 2) * 16 * NCB * 3 / 2 : 16 * NJ * 16 * NCB;
 
 // The three bf16 terms of x: 8 bits each by truncation, so hi + mid + lo is x
-// exactly; infinities and NaN stay in hi alone.
+// exactly (from 2^-110 up); infinities and NaN stay in hi alone.
 __device__ __forceinline__ void split3(float x, uint16_t (&t)[3]) {
     const uint32_t u = __float_as_uint(x);
     const float r1 = x - __uint_as_float(u & 0xffff0000u);
@@ -586,7 +587,7 @@ __device__ __forceinline__ void stream_block(int64_t id, int64_t N, int per, int
 }
 
 // One workgroup per (block of `wg_tokens` tokens, stream, slice of 16 NCB
-// output columns); wave w takes the 16-token tiles w, w + 4, ..  Rows of up to
+// output columns); wave w takes the 16-token tiles w, w + NW, ..  Rows of up to
 // 128 values are loaded as whole rows a tile ahead; longer ones straight in
 // the operands' layout (their turn would take 64 KB of LDS).
 template <typename TIn, int NJ, int NCB, bool kB16, int NW>

@@ -1001,13 +1001,16 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
     RACE_TRY(marks->mark(stream));
     const float* fwd_rec = fwd_records;
     if (!fwd_rec && !whole_streams) {
-        if (short_prefixes(p))  // the forward's own records, bit for bit
+        // Short prefixes and the narrow sums are the forward's own records, bit for
+        // bit (but for a bf16 forward with RACE_KERNEL_MFMA and one that advances a
+        // carried state in place, which take tile sums and a scan).
+        if (short_prefixes(p))
             RACE_TRY(launch_prefix_records(probsK, V, fwd_ws, p, stream));
         else if (direct_sums_supported(p.S, p.d) && p.tile % 64 == 0)
             RACE_TRY(launch_tile_sums_direct(probsK, V, fwd_ws, p, stream));
         else if (mfma_causal_supported(p.S, p.d))
             RACE_TRY(launch_tile_sums_mfma(probsK, V, fwd_ws, p, stream));
-        else if (narrow_causal(p, kernel))  // the forward's own records, bit for bit
+        else if (narrow_causal(p, kernel))
             RACE_TRY(launch_nc_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         else
             RACE_TRY(launch_tile_outer_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));

@@ -1,8 +1,9 @@
 """Drop-in BatchedACE (src/race_baseline.py:21-52) running the op on MI355X.
 
 Same constructor and forward signature as the reference module.  The whole
-forward is one op, ModuleRaceFunction, and the output permute of line 52 (a
-view): the permutes of lines 35-40 are one copy kernel for the three inputs.
+forward is one op, ModuleRaceFunction: the permutes of lines 35-40 are one
+copy kernel for the three inputs, and the output has the strides of the permute
+of line 52.
 For the causal module the hashing of lines 41-44 (shared hash planes, tanh,
 corner softmax) and the hot span of lines 45-51 run in the same kernels, which
 hash the Q and K rows themselves (the reference's fused forward,
@@ -46,9 +47,8 @@ class BatchedACE(nn.Module):
         hashed = self.causal and hashed_supported(self.L, self.K, dk)
         own = getattr(self.bucket_probs, "__func__", None) is not _BUCKET_PROBS
         if not own and (hashed or not self.causal):
-            out = ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal),
-                                           torch.is_grad_enabled())
-            return out.permute(0, 1, 3, 2, 4)
+            return ModuleRaceFunction.apply(Khf, Vhf, Qhf, self.planes_T, self.L, self.K, bool(self.causal),
+                                            torch.is_grad_enabled())
         Kh2 = Khf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
         Qh2 = Qhf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)
         V2 = Vhf.permute(0, 1, 3, 2, 4).contiguous().view(N, T, dk)

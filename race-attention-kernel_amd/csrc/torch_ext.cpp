@@ -16,9 +16,9 @@
 //       -> (out, records or None, state or None, tile_tokens): the causal op
 //       with the hashing inside (race_hashed_fwd)
 //   module_forward(K, V, Q, planes_T, L, planes_per_table, causal, need_k, need_v, need_q)
-//       -> (out [M, B, H, T, d], saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
+//       -> (out, saved, tile_tokens): BatchedACE.forward on [M, B, T, H, d] rows
 //   module_backward(grad_out, saved, L, planes_per_table, causal, tile_tokens,
-//       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None; grad_out [M, B, H, T, d]
+//       need_k, need_v, need_q) -> (dK, dV, dQ) rows or None
 //   hashed_supported(L, K, d) -> bool
 //   select_tile_tokens(N, T, L, R, d, bf16, causal, tile_tokens=0, kernel=0) -> int
 //   shape_supported(L, R, d) -> (supported, has_mfma)
@@ -576,9 +576,10 @@ int64_t select_tile_tokens(int64_t N, int64_t T, int64_t L, int64_t R, int64_t d
 
 // BatchedACE.forward (src/race_baseline.py:34-52) for K, V, Q [M, B, T, H, d]:
 // the heads' rows as streams, the hashing, and the op (causal: with the
-// hashing inside).  Returns the output [M, B, H, T, d] (no view: what a custom
-// autograd function returns as one may not be changed in place; the module
-// permutes it), and with a gradient to come what module_backward reads for it:
+// hashing inside).  Returns the output [M, B, T, H, d] in the strides of the
+// module's permute (but no view: what a custom autograd function returns as one
+// may not be changed in place), and with a gradient to come what
+// module_backward reads for it:
 // (V, K, Q rows, planes, tile records) and the records' tile length, or (V
 // rows, probsK, probsQ, state, then for K's and Q's gradients planes_T and the
 // rows of each that has one).
@@ -610,17 +611,17 @@ std::tuple<at::Tensor, std::vector<at::Tensor>, int64_t> module_forward(const at
         if (need_k) saved.push_back(rows[0]);
         if (need_q) saved.push_back(rows[1]);
     }
-    return {at::_unsafe_view(out, {M, B, H, T, d}), saved, tile};
+    out.as_strided_({M, B, T, H, d}, {B * H * T * d, H * T * d, d, T * d, 1});
+    return {out, saved, tile};
 }
 
 // Gradients of module_forward's rows [N, T, d] (None where not asked for) for
-// the upstream gradient [M, B, H, T, d] of the output (dense once its heads are
-// permuted back, where the module's output had a dense gradient).
+// the upstream gradient [M, B, T, H, d] of the output.
 std::tuple<c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>> module_backward(
     const at::Tensor& grad_out, const std::vector<at::Tensor>& saved, int64_t L, int64_t Kp, bool causal, int64_t tile,
     bool need_k, bool need_v, bool need_q) {
     const at::Tensor& V = saved[0];
-    const at::Tensor g = streams_of({grad_out.to(V.scalar_type()).permute({0, 1, 3, 2, 4})})[0].view(V.sizes());
+    const at::Tensor g = streams_of({grad_out.to(V.scalar_type())})[0].view(V.sizes());
     c10::optional<at::Tensor> dq, dk, dv;
     at::Tensor pT, K, Q;
     if (causal) {

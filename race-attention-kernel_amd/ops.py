@@ -253,9 +253,9 @@ def race_fused_fwd_hashed(K: torch.Tensor, Q: torch.Tensor, V: torch.Tensor, pla
 
 class ModuleRaceFunction(torch.autograd.Function):
     """BatchedACE.forward as one op: heads to streams, hashing and the op, and
-    their gradients, each direction one call into the binding.  The output is
-    [M, B, H, T, d]; the module permutes it outside, so that it may be changed
-    in place (the output of a custom function that is a view may not).
+    their gradients, each direction one call into the binding.  The output has
+    the strides of the module's permute but is no view, so that it may be changed
+    in place (a view out of a custom function may not).
 
     What it saves is what the separate ops save: the rows, the planes, and the
     forward's tile records (causal) or the probabilities and the state; the

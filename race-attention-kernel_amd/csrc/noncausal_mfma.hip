@@ -34,11 +34,12 @@
 //
 // Measured against the vector-ALU kernels (noncausal_v4.hip), S = d = 64,
 // kernel times in us, reduction / map / query side / key side:
-//   fp32, N = 384, T = 1024: 56 / 66 / 110 / 116 -> 37 / 47 / 66 / 81, at 5.4,
-//     4.3, 4.6 and 5.0 TB/s of tokens: bound by memory (the query side's two
-//     products alone are 41 us of fp32 matrix instructions);
+//   fp32, N = 384, T = 1024: 50 / 62 / 101 / 107 -> 36 / 44 / 61 / 81, at 5.6,
+//     4.6, 5.0 and 5.0 TB/s of tokens: bound by memory (the query side's two
+//     products alone are 41 us of fp32 matrix instructions); 44 for the
+//     reduction where no token is left in a cache by the call before;
 //   bf16, N = 192, T = 577: 20 + 10 (reduce) / 41 / 41 + 7 (finalize) / 41
-//     -> 10 / 9 / 14 / 14: launches of one workgroup per stream, bound by the
+//     -> 9 / 11 / 13 / 15: launches of one workgroup per stream, bound by the
 //     latency of staging, the loop's few steps and the launch itself.
 // Other widths (S 12 .. 256, d 20 .. 128) ran 1.2x (100 x 36, fp32) to 9x.
 #include <algorithm>

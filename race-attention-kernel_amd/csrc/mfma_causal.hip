@@ -168,15 +168,19 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_mfma_kernel(
 // fill the register file: two waves per SIMD then share the CU's work).
 //
 // kFused (short sequences, short_prefixes): the workgroup first sums the tokens
-// before its tile (quad_sums) into its record, and a workgroup past the last
-// tile sums every token into the state when it is asked for: one launch instead
-// of three.  Its records are `prefixes`, which it writes; `records` stays a
-// read-only operand of the unfused pass.
-template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, bool kFused = false>
+// before its tile (quad_sums) into its record: one launch instead of three.  Its
+// records are `prefixes`, which it writes; `records` stays a read-only operand
+// of the unfused pass.  The state, when it is asked for, comes from a workgroup
+// past the last tile that sums every token (kShort), or from the last tile's:
+// what it carries at its end, B as it stands and A from fp32 sums of its keys
+// (kShortLast).
+enum Fused { kThreeLaunches, kShort, kShortLast };
+template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, int kMode = kThreeLaunches>
 __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v,
     TIn* __restrict__ out, const float* __restrict__ records, int64_t T, int tile, int64_t tiles,
     int64_t rec, float* prefixes, const float* init, float* state) {
+    constexpr bool kFused = kMode != kThreeLaunches;
     using G = Geo<TIn, S, D, C, NW, kPrecise>;
     using PS = typename G::PS;
     using PK = typename G::PK;
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     const int tid = threadIdx.x, l = tid & 63, g = l >> 4, lr = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t n = blockIdx.y, ti = blockIdx.x;
-    if constexpr (kFused) {
+    if constexpr (kMode == kShort) {
         if (ti == tiles) {
             quad_sums<TIn>(k + n * T * S, v + n * T * D, int(T), int(T), reinterpret_cast<float*>(lds),
                            state + n * (S * D + S), init ? init + n * (S * D + S) : nullptr);
@@ -454,6 +458,30 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     }
     __syncthreads();
     if (r0 > 0) OT::template flush<kStoreP, G::kT>(Os, or_, r0 - C);
+    if constexpr (kMode == kShortLast) {
+        if (ti != tiles - 1) return;
+        float* st_p = state + n * (S * D + S);
+#pragma unroll
+        for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) st_p[(16 * sb + 4 * g + rr) * D + 16 * w + lr] = b0[sb][0][rr];
+        // Keys of rows 16 i + 4 w + g, columns 4 lr ..; the row groups, then the
+        // waves in order (the W tile is free).
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int row = 4 * w + g; row < rows; row += 16)
+            a += load_q4<TIn, kPolicyDefault>(kr, (row * S + 4 * lr) * int(sizeof(TIn)));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            a[c] += __shfl_xor(a[c], 16);
+            a[c] += __shfl_xor(a[c], 32);
+        }
+        float* part = reinterpret_cast<float*>(Ws);
+        if (g == 0) *reinterpret_cast<f32x4*>(part + 64 * w + 4 * lr) = a;
+        __syncthreads();
+        if (tid < S)
+            st_p[S * D + tid] = rec_p[S * D + tid] + (((part[tid] + part[64 + tid]) + part[128 + tid]) + part[192 + tid]);
+    }
 }
 
 // K1 alone: the register-direct kernel where it applies, else the workgroup one.
@@ -481,14 +509,27 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     hipError_t err = hipSuccess;
     if constexpr (S == 64 && D == 64) {
         // One launch.  (A state must not be written over the carried one while
-        // other workgroups still read it.)
+        // other workgroups still read it.)  A state by workgroups of its own where
+        // all are resident at once (two per CU), by the last tile's otherwise.
+        // Measured with the state, against three launches, fp32: own workgroups N =
+        // 8, T = 512 14.9 -> 12.4 us, but N = 128, T = 512 30.5 -> 36.2 and N = 1024, T
+        // = 512 153 -> 188; by the last tile 31 and 118.  (One kernel for both would
+        // cost calls without the state 3%.)
+        const bool resident = p.N * (p.tiles + 1) <= 512;
         if (short_prefixes(p) && (!state || state != p.init)) {
             constexpr size_t kQuad = kQuadLdsFloats * sizeof(float);
             constexpr size_t kLds = size_t(GO::kOutputLds) > kQuad ? size_t(GO::kOutputLds) : kQuad;
-            const dim3 fused(unsigned(p.tiles + (state ? 1 : 0)), unsigned(p.N));
-            causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, true><<<fused, GO::kT, kLds, stream>>>(
-                static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
-                static_cast<TIn*>(out), nullptr, p.T, p.tile, p.tiles, p.rec, records, p.init, state);
+            const dim3 fused(unsigned(p.tiles + (state && resident ? 1 : 0)), unsigned(p.N));
+            auto launch = [&](auto mode) {
+                causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, decltype(mode)::value>
+                    <<<fused, GO::kT, kLds, stream>>>(
+                        static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
+                        static_cast<TIn*>(out), nullptr, p.T, p.tile, p.tiles, p.rec, records, p.init, state);
+            };
+            if (state && !resident)
+                launch(std::integral_constant<int, kShortLast>{});
+            else
+                launch(std::integral_constant<int, kShort>{});
             if ((err = hipGetLastError()) != hipSuccess) return err;
             return marks ? marks->mark(stream) : hipSuccess;
         }

@@ -2,7 +2,8 @@
 tokens before their own tile.
 
 Around the rule's edges (the last tile starting at 512 tokens, six tiles or
-512 workgroups), against fp64: outputs, the prefix records, the state, a
+512 workgroups, the state from workgroups of its own or from the last tile's),
+against fp64: outputs, the prefix records, the state, a
 carried state (also advanced in place, which takes the three launches), and
 the backward from the saved records against the one that recomputes them.
 """
@@ -21,7 +22,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kernel", ["auto", "mfma_wg", "mfma_precise"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("N, T, tile", [(1, 1, 0), (2, 64, 0), (3, 65, 0), (2, 512, 0), (2, 576, 64), (2, 577, 64),
-                                        (2, 641, 128), (1, 1500, 2048), (64, 512, 64), (65, 500, 64), (86, 384, 64)])
+                                        (2, 641, 128), (1, 1500, 2048), (64, 512, 64), (65, 500, 64), (86, 384, 64),
+                                        (300, 64, 0), (520, 33, 0), (130, 300, 0), (257, 600, 512)])
 def test_outputs_records_and_states(race, ext, oracle, cuda, kernel, dtype, N, T, tile):
     say("short", kernel, dtype, N, T, tile)
     q, k, v = race.make_inputs(N, T, 4, 16, 64, seed=T + N, dtype=dtype)

@@ -420,14 +420,30 @@ hipError_t launch_t(const void* x, const float* planes_T, const void* dprobs, vo
 // Rows are loaded as 16- or 8-byte groups of four values (d_k a multiple of 4)
 // and probability rows as whole 16-byte chunks, from 16-byte aligned arrays;
 // K = 1 (no quads of corners), K = 7, 8 (32 and 64 quads of corners unrolled
-// per lane) and every other row layout take the row-per-thread kernels.  Within
-// those forms these kernels were faster in every case measured (500 to 400000
-// rows, both dtypes, K = 2 .. 6, d_k = 32 .. 128): forward 1.2x (K = 5, d_k =
-// 64, fp32) to 7x, gradient 4x to 22x.
-bool hash_rows_supported(const void* x, const void* probs, const void* dx, int dk, int L, int K, int dtype) {
+// per lane) and every other row layout take the row-per-thread kernels.
+//
+// So do few tables of narrow rows: a set (8 tables of 2 planes, 4 of more) costs
+// the same however many of its tables there are, and 16 or fewer columns as much
+// as 64, while a thread of the row-per-thread kernels does only what a row
+// needs.  Measured against those, fp32, 200000 / 800000 rows, forward: L = 1,
+// K = 4, d_k = 32 1.06 / 1.04 of their time, 40 0.86 / 0.90; L = 2 16 0.96 / 1.04,
+// 20 0.92 / 1.02; L = 4, K = 2 20 1.04 / 1.11, 24 0.99 / 1.06.  Gradient: L = 1, K = 3
+// 12 0.98 / 1.27, 16 0.83 / 1.07; L = 2, K = 3 4 0.80 / 0.97.  bf16 rows cost these
+// kernels less (L = 1, K = 4, d_k = 24 1.06 / 1.09, 32 0.98 / 0.99).  Up to 20000
+// rows these kernels took 0.6 to 0.95 of the time there too, but a row's result
+// does not depend on how many there are.  Within the rest they were faster: at
+// d_k = 64, K = 2 .. 6, forward 0.2 to 0.95 of the time, gradient 0.04 to 0.4 (past
+// 800000 rows of one table of 64 or three of 32 corners, fp32, bound by the
+// writes, forward up to 1.16).
+bool hash_rows_supported(const void* x, const void* probs, const void* dx, int dk, int L, int K, int dtype,
+                         bool gradient) {
     const int es = dtype == RACE_BF16 ? 2 : 4;
-    return K >= 2 && K <= 6 && dk % 4 == 0 && ((L << K) * es) % 16 == 0 && aligned(x) && aligned(probs) &&
-           aligned(dx);
+    if (K < 2 || K > 6 || dk % 4 != 0 || ((L << K) * es) % 16 != 0 || !aligned(x) || !aligned(probs) || !aligned(dx))
+        return false;
+    const int set = K == 2 ? 8 : 4;
+    if (gradient) return !(K <= 4 && 4 * L <= set && dk <= 12);
+    const int columns = (dtype == RACE_BF16 ? 6 : 8) + (K == 2 ? 2 : 0);
+    return !(2 * L <= set && dk <= 32 && L * dk <= columns * set);
 }
 
 hipError_t launch_hash_rows(const void* x, const float* planes_T, const void* dprobs, void* out, int64_t rows,

@@ -298,7 +298,7 @@ constexpr int64_t kLaunchRows = int64_t(1) << 30;
 
 hipError_t hash_probs_rows(const void* x, const float* planes_T, void* probs, int64_t rows,
                            int dk, int L, int K, int dtype, hipStream_t stream) {
-    if (hash_rows_supported(x, probs, probs, dk, L, K, dtype))
+    if (hash_rows_supported(x, probs, probs, dk, L, K, dtype, false))
         return launch_hash_rows(x, planes_T, nullptr, probs, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kHashRows - 1) / kHashRows));
     const size_t lds = hash_lds_bytes(dk, L, K);
@@ -332,7 +332,7 @@ hipError_t hash_probs_rows(const void* x, const float* planes_T, void* probs, in
 
 hipError_t hash_probs_bwd_rows(const void* x, const float* planes_T, const void* dprobs, void* dx,
                                int64_t rows, int dk, int L, int K, int dtype, hipStream_t stream) {
-    if (hash_rows_supported(x, dprobs, dx, dk, L, K, dtype))
+    if (hash_rows_supported(x, dprobs, dx, dk, L, K, dtype, true))
         return launch_hash_rows(x, planes_T, dprobs, dx, rows, dk, L, K, dtype, stream);
     const dim3 grid(unsigned((rows + kThreads - 1) / kThreads));
     const int tier = lk_tier(L * K);

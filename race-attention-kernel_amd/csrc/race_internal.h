@@ -397,7 +397,8 @@ hipError_t launch_hash_probs_bwd(const void* x, const float* planes_T, const voi
 // The same two on the matrix cores, 16 rows per wave (hash_rows.hip): whether
 // these arrays and this shape have kernels there, and the launch (dprobs null:
 // probs into `out`; else dx into `out`).
-bool hash_rows_supported(const void* x, const void* probs, const void* dx, int dk, int L, int K, int dtype);
+bool hash_rows_supported(const void* x, const void* probs, const void* dx, int dk, int L, int K, int dtype,
+                         bool gradient);
 hipError_t launch_hash_rows(const void* x, const float* planes_T, const void* dprobs, void* out, int64_t rows,
                             int dk, int L, int K, int dtype, hipStream_t stream);
 

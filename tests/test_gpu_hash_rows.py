@@ -2,9 +2,10 @@
 
 Every slot layout (2 to 6 planes per table, tables that fill a lane group's
 slots or leave some empty, one or more sets of tables), row lengths that are
-not multiples of 16, and row counts around the 16-row groups and the 128-row
-workgroups, against the reference's composition (src/race_baseline.py:41-44)
-and its autograd gradient in fp64 on the CPU.
+not multiples of 16, row counts around the 16-row groups and the 128-row
+workgroups, and few tables of narrow rows, which take the row-per-thread
+kernels in one direction or both, against the reference's composition
+(src/race_baseline.py:41-44) and its autograd gradient in fp64 on the CPU.
 """
 from __future__ import annotations
 
@@ -29,7 +30,8 @@ def hash64(x, planes_T, L, K):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dk, L, K", [(64, 4, 4), (64, 2, 2), (60, 9, 2), (64, 4, 3), (20, 21, 3), (128, 8, 4),
-                                      (68, 5, 4), (128, 8, 5), (64, 3, 5), (64, 1, 6), (100, 4, 6), (4, 3, 4)])
+                                      (68, 5, 4), (128, 8, 5), (64, 3, 5), (64, 1, 6), (100, 4, 6), (4, 3, 4),
+                                      (32, 1, 4), (36, 1, 4), (16, 2, 3), (20, 4, 2), (12, 1, 3), (16, 1, 3), (28, 1, 5)])
 @pytest.mark.parametrize("rows", [1, 17, 128, 333])
 def test_rows_and_gradients(race, cuda, dtype, dk, L, K, rows):
     say("hash rows", dtype, dk, L, K, rows)

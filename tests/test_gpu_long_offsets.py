@@ -106,9 +106,9 @@ def skip_unless_free(nbytes):
 
 def test_hashing_of_more_than_2_to_the_31_rows(race, cuda):
     # More rows than one launch of the 16-row kernels holds threads for.
-    dk, L, K = 4, 2, 2
+    dk, L, K = 4, 6, 2
     rows = 2 ** 31 + 200
-    skip_unless_free(rows * 2 * 2 * (dk + L * (1 << K)))
+    skip_unless_free(rows * 2 * (2 * dk + L * (1 << K)))
     say("hash rows", rows)
     gen = torch.Generator(device=cuda).manual_seed(31)
     planes_T = torch.randn(dk, L * K, generator=gen, device=cuda)

@@ -175,7 +175,9 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void tile_sums_mfma_kernel(
 // what it carries at its end, B as it stands and A from fp32 sums of its keys
 // (kShortLast).
 enum Fused { kThreeLaunches, kShort, kShortLast };
-template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, int kMode = kThreeLaunches>
+// kPast (bf16): Q and the output go past the caches (past_caches).
+template <typename TIn, int S, int D, int C, int kMinBlocks, int NW, bool kPrecise, int kMode = kThreeLaunches,
+          bool kPast = false>
 __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v,
     TIn* __restrict__ out, const float* __restrict__ records, int64_t T, int tile, int64_t tiles,
@@ -203,12 +205,6 @@ __global__ __launch_bounds__(64 * NW, kMinBlocks) void causal_output_mfma_kernel
     constexpr bool kQStage = G::kQStage;
     constexpr int kQChunks = C * QT::kChunks;
     constexpr int kQPer = (kQChunks + G::kT - 1) / G::kT;
-    // S = d = 64: Q and the output go past the caches, which hold the K and V
-    // rows the tile sums left for this pass (cache_kept_rows).  bf16, N = 8, T =
-    // 131072: 97 us, 89 with Q and 84 with both.  The other bf16 shapes, whose
-    // tile sums leave nothing, keep the default (S = 256, d = 128 ran 997 -> 1015
-    // us with nontemporal stores).
-    constexpr bool kPast = S == 64 && D == 64;
     constexpr int kStoreP = std::is_same<TIn, float>::value ? kOutWgStorePolicyF32 : kPast ? kPolicyStream : kOutStorePolicy;
     constexpr int kQP = std::is_same<TIn, float>::value ? kOutQPolicyF32 : kPast ? kPolicyStream : kOutQPolicy;
     // Sub-chunks of operands in flight in registers ahead of the one in LDS.
@@ -500,6 +496,19 @@ hipError_t launch_sums_family(const void* k, const void* v, float* records, cons
     return hipGetLastError();
 }
 
+// bf16, S = d = 64: whether Q and the output go past the caches, which hold the
+// K and V rows the tile sums left for the output pass (cache_kept_rows): from
+// 201 MB of Q, K, V and output on.  Smaller calls fit the memory-side cache
+// whole, where the next launch (the caller's, or the next call's sums) finds
+// the output.  Measured, whole forward, inputs that change, default and past: N =
+// 8, T = 131072 (537 MB) 166 and 149 us, T = 65536 (268 MB) 85 and 80, T = 32768
+// 50.2 and 50.2; N = 100, T = 512 (26 MB) 24.4 and 26.7.  The other bf16 shapes,
+// whose tile sums leave nothing, keep the default (S = 256, d = 128 ran 997 ->
+// 1015 us with nontemporal stores).
+bool past_caches(const Problem& p) {
+    return p.dtype == RACE_BF16 && p.S == 64 && p.d == 64 && p.N * p.T * 4 * 64 * 2 >= int64_t(3) << 26;
+}
+
 template <typename TIn, bool kPrecise, int S, int D, int C, int kMinBlocks, int NW = 4>
 hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void* out, float* records,
                               float* state, const Problem& p, hipStream_t stream, Marks* marks) {
@@ -507,6 +516,11 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     static_assert(GO::kOutputLds <= 160 * 1024, "gfx950 gives a workgroup at most 160 KB of LDS");
     const dim3 grid(unsigned(p.tiles), unsigned(p.N));
     hipError_t err = hipSuccess;
+    // Kernels that send Q and the output past the caches: bf16 at S = d = 64.
+    constexpr bool kHasPast = S == 64 && D == 64 && std::is_same<TIn, bf16_t>::value;
+    using Default = std::false_type;
+    using Past = std::integral_constant<bool, kHasPast>;
+    const bool past = past_caches(p);
     if constexpr (S == 64 && D == 64) {
         // One launch.  (A state must not be written over the carried one while
         // other workgroups still read it.)  A state by workgroups of its own where
@@ -520,16 +534,19 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
             constexpr size_t kQuad = kQuadLdsFloats * sizeof(float);
             constexpr size_t kLds = size_t(GO::kOutputLds) > kQuad ? size_t(GO::kOutputLds) : kQuad;
             const dim3 fused(unsigned(p.tiles + (state && resident ? 1 : 0)), unsigned(p.N));
-            auto launch = [&](auto mode) {
-                causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, decltype(mode)::value>
+            auto launch = [&](auto mode, auto to) {
+                causal_output_mfma_kernel<TIn, S, D, C, 2, NW, kPrecise, decltype(mode)::value, decltype(to)::value>
                     <<<fused, GO::kT, kLds, stream>>>(
                         static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
                         static_cast<TIn*>(out), nullptr, p.T, p.tile, p.tiles, p.rec, records, p.init, state);
             };
-            if (state && !resident)
-                launch(std::integral_constant<int, kShortLast>{});
+            using Own = std::integral_constant<int, kShort>;
+            using Last = std::integral_constant<int, kShortLast>;
+            const bool last = state && !resident;
+            if (past)
+                last ? launch(Last{}, Past{}) : launch(Own{}, Past{});
             else
-                launch(std::integral_constant<int, kShort>{});
+                last ? launch(Last{}, Default{}) : launch(Own{}, Default{});
             if ((err = hipGetLastError()) != hipSuccess) return err;
             return marks ? marks->mark(stream) : hipSuccess;
         }
@@ -539,9 +556,13 @@ hipError_t launch_mfma_family(const void* q, const void* k, const void* v, void*
     if (marks && (err = marks->mark(stream)) != hipSuccess) return err;
     if ((err = launch_tile_scan(records, state, p, stream)) != hipSuccess) return err;
     if (marks && (err = marks->mark(stream)) != hipSuccess) return err;
-    causal_output_mfma_kernel<TIn, S, D, C, kMinBlocks, NW, kPrecise><<<grid, GO::kT, GO::kOutputLds, stream>>>(
-        static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
-        static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, nullptr, nullptr, nullptr);
+    auto launch = [&](auto to) {
+        causal_output_mfma_kernel<TIn, S, D, C, kMinBlocks, NW, kPrecise, kThreeLaunches, decltype(to)::value>
+            <<<grid, GO::kT, GO::kOutputLds, stream>>>(
+                static_cast<const TIn*>(q), static_cast<const TIn*>(k), static_cast<const TIn*>(v),
+                static_cast<TIn*>(out), records, p.T, p.tile, p.tiles, p.rec, nullptr, nullptr, nullptr);
+    };
+    past ? launch(Past{}) : launch(Default{});
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (marks) return marks->mark(stream);

@@ -97,3 +97,18 @@ def test_every_launch_is_marked_once(race, cuda, T, tile, fwd, bwd):
                                         nbytes, stream.cuda_stream, handles)
     assert (status, n) == (0, bwd + 1)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T, tile", [(400, 512), (600, 128), (1100, 512)])
+def test_large_calls_give_the_bits_of_small_ones(race, ext, cuda, T, tile):
+    # From 201 MB of bf16 tensors on Q and the output go past the caches (one
+    # launch of one tile, one of five, three launches): other instructions, the
+    # same values.
+    N = (3 << 26) // (T * 512) + 1
+    say("past the caches", N, T, tile)
+    q, k, v = race.make_inputs(N, T, 4, 16, 64, seed=T, dtype=torch.bfloat16, device=cuda)
+    big = ext.forward(q, k, v, True, tile, 0, False)[0]
+    for n in (0, N - 5):
+        small = ext.forward(*(x[n:n + 5].clone() for x in (q, k, v)), True, tile, 0, False)[0]
+        assert torch.equal(big[n:n + 5], small)
+    assert torch.equal(ext.forward(q, k, v, True, tile, 0, True)[0], big)

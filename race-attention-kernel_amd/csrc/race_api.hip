@@ -1003,8 +1003,12 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
     if (!fwd_rec && !whole_streams) {
         // Short prefixes and the narrow sums are the forward's own records, bit for
         // bit (but for a bf16 forward with RACE_KERNEL_MFMA and one that advances a
-        // carried state in place, which take tile sums and a scan).
-        if (short_prefixes(p))
+        // carried state in place, which take tile sums and a scan).  With seven tiles
+        // or more the prefixes' launch is the shorter only while every workgroup has a
+        // CU of its own: fp32, N = 8, T = 512 (8 tiles) 26.2 -> 25.6 us for the whole
+        // backward, but N = 64 44.7 -> 51.3.
+        const bool prefixes = short_prefixes(p) && (p.tiles <= 6 || p.N * p.tiles <= 256);
+        if (prefixes)
             RACE_TRY(launch_prefix_records(probsK, V, fwd_ws, p, stream));
         else if (direct_sums_supported(p.S, p.d) && p.tile % 64 == 0)
             RACE_TRY(launch_tile_sums_direct(probsK, V, fwd_ws, p, stream));
@@ -1015,7 +1019,7 @@ race_status causal_bwd_impl(const void* probsQ, const void* probsK, const void* 
         else
             RACE_TRY(launch_tile_outer_sums(probsK, V, fwd_ws, p, p.S, p.d, stream));
         RACE_TRY(marks->mark(stream));
-        if (!short_prefixes(p)) {
+        if (!prefixes) {
             RACE_TRY(launch_tile_scan(fwd_ws, nullptr, p, stream));
             RACE_TRY(marks->mark(stream));
         }

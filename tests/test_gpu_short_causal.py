@@ -72,6 +72,18 @@ def test_saved_records_and_recomputed_ones_give_the_same_bits(race, ext, cuda, d
     assert all(torch.equal(a, b) for a, b in zip(saved, again))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_recomputed_records_of_many_short_streams(race, ext, cuda, dtype):
+    # 8 tiles of 64 over more workgroups than CUs: tile sums and a scan, other
+    # sums of the same records.
+    q, k, v, g = race.make_inputs(40, 512, 4, 16, 64, seed=8, dtype=dtype, device=cuda, grad_out=True)
+    _, records, used = ext.forward_with_records(q, k, v, 64, 0)
+    saved = ext.causal_backward(q, k, v, g, True, True, True, used, 0, records)
+    again = ext.causal_backward(q, k, v, g, True, True, True, used, 0, None)
+    for a, b in zip(saved, again):
+        assert per_stream_rel_err(to_np(a), to_np(b)) <= (BF16_TOL if dtype == torch.bfloat16 else FP32_TOL)
+
+
 @pytest.mark.parametrize("T, tile, fwd, bwd", [(512, 64, 1, 4), (576, 64, 1, 4), (577, 64, 3, 5)])
 def test_every_launch_is_marked_once(race, cuda, T, tile, fwd, bwd):
     # An event before the first launch and after every one, none for launches
